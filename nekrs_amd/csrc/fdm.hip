@@ -535,51 +535,56 @@ __global__ __launch_bounds__(FdmCfg<NQ>::BLOCK) void fdm_kernel(
 // ASM overlap exchange (extended gather-scatter + postFDM.c:3-155): each node
 // on the second layer from a face with a neighbour gets (own + neighbour) -
 // own of the overlap results there, in the order k faces, j faces, i faces;
-// then the Schwarz weight.  One thread per (j, k) row of i values.
+// then the Schwarz weight.  One block per element and one thread per node, so
+// that the restricted results, the weights and Su are read and written
+// coalesced and the face maps are scalar loads.  Bound by the chain of loads
+// (face map, then the two overlap values): the six faces' loads are issued
+// together without branches, at an address of the element's own where a lane
+// has no value to fetch (one thread per row of NQ nodes, branching per face:
+// one order-5 ASM application on 5 814 elements 40.8 us, this form 32.4 us).
+template <int NQ> struct PostCfg {
+  static constexpr int NP = NQ * NQ * NQ;
+  static constexpr int BLOCK = NP >= 256 ? 256 : (NP + 63) / 64 * 64;
+};
 template <typename T, int NQ>
-__global__ __launch_bounds__(256) void fdm_post_kernel(int E, const T *__restrict__ box,
-                                                       const T *__restrict__ gout,
-                                                       const int4 *__restrict__ smap,
-                                                       const T *__restrict__ wts, T *__restrict__ Su,
-                                                       const uint32_t *__restrict__ mbits)
+__global__ __launch_bounds__(PostCfg<NQ>::BLOCK) void fdm_post_kernel(
+    int E, const T *__restrict__ box, const T *__restrict__ gout, const int4 *__restrict__ smap,
+    const T *__restrict__ wts, T *__restrict__ Su, const uint32_t *__restrict__ mbits)
 {
-  constexpr int NP = NQ * NQ * NQ, NQ2 = NQ * NQ;
-  const int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (row >= (int64_t)E * NQ2) return;
-  const int64_t e = row / NQ2;
-  const int r = (int)(row - e * NQ2), j = r % NQ, k = r / NQ;
-  const int64_t base = e * NP + (int64_t)r * NQ;
-  const T *ge = gout + e * 6 * NQ2;
-  T v[NQ];
+  constexpr int NP = NQ * NQ * NQ, NQ2 = NQ * NQ, BLOCK = PostCfg<NQ>::BLOCK;
+  const int e = blockIdx.x;
+  const int64_t base = (int64_t)e * NP;
+  const T *ge = gout + (int64_t)e * 6 * NQ2;
+  const uint32_t *mb = mbits ? mbits + (int64_t)e * ((NP + 31) / 32) : nullptr;
+  int4 sm[6];
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) v[i] = box[base + i];
-  // overlap value at face point (uu, vv) of face f: (own + neighbour) - own
-  auto ov = [&](int f, int uu, int vv) -> T {
-    const int4 sm = smap[e * 6 + f];
-    if (sm.x < 0) return T(0);
-    const T own = ge[f * NQ2 + vv * NQ + uu];
-    return (own + gout[sm.x + uu * sm.y + vv * sm.z]) - own;
-  };
-  if (k == 1)
+  for (int f = 0; f < 6; ++f) sm[f] = smap[(int64_t)e * 6 + f];
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) v[i] += ov(0, i, j);
-  if (k == NQ - 2)
+  for (int t = 0; t < (NP + BLOCK - 1) / BLOCK; ++t) {
+    const int n = t * BLOCK + (int)threadIdx.x;
+    if (n >= NP) break;
+    const int i = n % NQ, j = (n / NQ) % NQ, k = n / NQ2;
+    T v = box[base + n];
+    const T w = wts[base + n];
+    // faces whose overlap layer holds the node, and the face point (uu, vv) there
+    const bool layer[6] = {k == 1, j == 1, i == NQ - 2, j == NQ - 2, i == 1, k == NQ - 2};
+    const int uu[6] = {i, i, j, i, j, i}, vv[6] = {j, k, k, k, k, j};
+    bool on[6];
+    T own[6], nb[6];
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) v[i] += ov(5, i, j);
-  if (j == 1)
+    for (int f = 0; f < 6; ++f) {
+      on[f] = layer[f] && sm[f].x >= 0;
+      own[f] = ge[on[f] ? f * NQ2 + vv[f] * NQ + uu[f] : 0];
+      nb[f] = gout[on[f] ? sm[f].x + uu[f] * sm[f].y + vv[f] * sm[f].z : e * 6 * NQ2];
+    }
+    constexpr int order[6] = {0, 5, 1, 3, 4, 2};
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) v[i] += ov(1, i, k);
-  if (j == NQ - 2)
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) v[i] += ov(3, i, k);
-  v[1] += ov(4, j, k);
-  v[NQ - 2] += ov(2, j, k);
-  // masked nodes (in no gather-scatter row) stored as zero
-  const uint32_t *mb = mbits ? mbits + e * ((NP + 31) / 32) : nullptr;
-#pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    const int n = r * NQ + i;
-    Su[base + i] = (mb && ((mb[n >> 5] >> (n & 31)) & 1u)) ? T(0) : v[i] * wts[base + i];
+    for (int q = 0; q < 6; ++q) {
+      const int f = order[q];
+      if (on[f]) v += (own[f] + nb[f]) - own[f];   // overlap value: (own + neighbour) - own, 0 without a neighbour
+    }
+    // masked nodes (in no gather-scatter row) stored as zero
+    Su[base + n] = (mb && ((mb[n >> 5] >> (n & 31)) & 1u)) ? T(0) : v * w;
   }
 }
 
@@ -1016,8 +1021,7 @@ template <typename T, int NQ>
 void launch_post_nq(int E, const T *box, const T *gout, const int4 *smap, const T *wts, T *Su,
                     const uint32_t *mbits, hipStream_t s)
 {
-  const int64_t rows = (int64_t)E * NQ * NQ;
-  fdm_post_kernel<T, NQ><<<(unsigned)((rows + 255) / 256), 256, 0, s>>>(E, box, gout, smap, wts, Su, mbits);
+  fdm_post_kernel<T, NQ><<<(unsigned)E, PostCfg<NQ>::BLOCK, 0, s>>>(E, box, gout, smap, wts, Su, mbits);
   NRS_LAUNCH_CHECK();
 }
 
