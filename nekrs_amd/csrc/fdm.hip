@@ -988,6 +988,211 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
   flush(prev);
 }
 
+// ---- FP32 variant: the six contractions on the FP32 matrix cores
+//
+// One element per wavefront, the box in one LDS buffer.  A contraction takes
+// the NL^2 rows (pencils) of the box 16 at a time: v_mfma_f32_16x16x4_f32 over
+// KS steps, row = lane % 16, contraction index KS (lane / 16) + step, which a
+// lane reads as KS consecutive floats (the 16 rows of a step start in distinct
+// banks).  The result, 16 rows by NL outputs, stays in the accumulators until
+// every row has been read and is then stored transposed over the same buffer,
+// output index first and the row pair after it, so the next contraction index is
+// again the fastest: X[k][j][i] -> T1[m][k][j] -> T2[n][m][k] -> T3[p][n][m] (times
+// invL) -> T4[i][p][n] -> T5[j][i][p] -> out[k][j][i].  FP32 operands and sums, as in the
+// one-thread-per-pencil form this replaced, which spent its time waiting for
+// scalar loads of the operators (100 each in six phases).  Order 7, 8000
+// elements: 47.3 -> 33 us a launch (counters: matrix cores busy 45 % of it, VALU
+// 25 %, the rest the loads at the start of each wave; a persistent wave that
+// loads the next element ahead, 1 to 5 blocks per CU, was 5-60 % slower).
+template <int NQ> struct FdmF32Cfg {
+  static constexpr int NL = NQ + 2;
+  static constexpr int NT = (NL * NL + 15) / 16;     // tiles of 16 rows
+  static constexpr int KS = (NL + 3) / 4;            // steps of 4 contraction indices
+  // plane stride: holds the NT tiles' results (16-byte aligned), and continues
+  // the rows' bank sequence from one plane to the next
+  static constexpr int PS0 = 16 * NT, PSR = (NL * NL) % 32 / 4 * 4;
+  static constexpr int PS = PS0 + ((PSR - PS0) % 32 + 32) % 32;
+  static constexpr int BOX = NL * PS;
+  static constexpr int WAVES = 4;
+  static constexpr int WAVES_PER_EU = (NQ == 7) ? 4 : (NQ <= 8) ? 5 : 3;   // the most without spills
+  static_assert(NL * NL - NL + 4 * KS <= PS0, "operand reads stay inside a plane's results");
+  static_assert(NL <= 12 && PS % 4 == 0, "one 16-wide tile of outputs, aligned rows");
+};
+
+template <int NQ, bool ASM>
+__global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kernel(
+    int E, const float *__restrict__ u, const float *__restrict__ S, const double *__restrict__ lam,
+    double2 helm, const int4 *__restrict__ gmap, float *__restrict__ out, float *__restrict__ gout,
+    const uint32_t *__restrict__ mbits)
+{
+  using C = FdmF32Cfg<NQ>;
+  constexpr int NL = C::NL, NT = C::NT, KS = C::KS, PS = C::PS, NP = NQ * NQ * NQ, NQ2 = NQ * NQ;
+  constexpr int RI = (NP + 63) / 64, RG = (NQ2 + 63) / 64, RL = (16 * NT + 63) / 64;
+  __shared__ __align__(16) float lds[C::WAVES][C::BOX];
+  __shared__ __align__(16) double lyzS[C::WAVES][16 * NT];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int e = __builtin_amdgcn_readfirstlane(blockIdx.x * C::WAVES + wv);
+  if (e >= E) return;                                // waves are independent: no block barrier below
+  float *X = lds[wv];
+  double *lyz = lyzS[wv];
+  auto at = [](int k, int j, int i) { return k * PS + j * NL + i; };
+  // box position of point (uu, vv) of face f's layer (0: ghost, 2: the second layer inside)
+  auto face_at = [&](int f, int uu, int vv, int d) {
+    switch (f) {
+      case 0: return at(d, vv + 1, uu + 1);
+      case 5: return at(NL - 1 - d, vv + 1, uu + 1);
+      case 1: return at(vv + 1, d, uu + 1);
+      case 3: return at(vv + 1, NL - 1 - d, uu + 1);
+      case 4: return at(vv + 1, uu + 1, d);
+      default: return at(vv + 1, uu + 1, NL - 1 - d);
+    }
+  };
+
+  // ---- loads: the element, its neighbours' second layers, operators, eigenvalues
+  const float *ue = u + (int64_t)e * NP;
+  float vi[RI], nb[6][RG], bf[3][KS], bb[3][KS];
+  double lx[KS], ly[RL], lz[RL];
+#pragma unroll
+  for (int t = 0; t < RI; ++t) {
+    const unsigned n = lane + 64 * t;
+    vi[t] = (n < NP) ? ue[n] : 0.f;
+  }
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    const int4 gm = gmap[(int64_t)e * 6 + f];
+#pragma unroll
+    for (int t = 0; t < RG; ++t) {
+      const int n = lane + 64 * t;
+      nb[f][t] = (gm.x >= 0 && n < NQ2) ? u[(unsigned)(gm.x + (n % NQ) * gm.y + (n / NQ) * gm.z)] : 0.f;
+    }
+  }
+  const float *Se = S + (int64_t)e * 3 * NL * NL;
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {   // forward B[l][m] = S[l][m], backward B[m][l] = S[l][m]; zero past the box
+      const int k = KS * g + s;
+      const bool ok = k < NL && c < NL;
+      bf[d][s] = ok ? Se[(unsigned)(d * NL * NL + k * NL + c)] : 0.f;
+      bb[d][s] = ok ? Se[(unsigned)(d * NL * NL + c * NL + k)] : 0.f;
+    }
+  const double *le = lam + (int64_t)e * 3 * NL;
+#pragma unroll
+  for (int t = 0; t < RL; ++t) {
+    const unsigned r = lane + 64 * t;   // row (p, n) of T3
+    ly[t] = (r < NL * NL) ? le[NL + r % NL] : 0.0;
+    lz[t] = (r < NL * NL) ? le[2 * NL + r / NL] : 0.0;
+  }
+#pragma unroll
+  for (int s = 0; s < KS; ++s) lx[s] = (KS * g + s < NL) ? le[(unsigned)(KS * g + s)] : 0.0;
+
+  // ---- the extended box (preFDM.c:16-96): zero (edges, corners, padding), interior, ghost faces
+  for (int n = lane; n < C::BOX / 4; n += 64) reinterpret_cast<float4 *>(X)[n] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int t = 0; t < RL; ++t)
+    if (lane + 64 * t < 16 * NT) lyz[lane + 64 * t] = ly[t] + lz[t];
+  wave_lds_sync();
+#pragma unroll
+  for (int t = 0; t < RI; ++t) {
+    const int n = lane + 64 * t;
+    if (n < NP) X[at(n / NQ2 + 1, (n / NQ) % NQ + 1, n % NQ + 1)] = vi[t];
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int f = 0; f < 6; ++f)
+#pragma unroll
+    for (int t = 0; t < RG; ++t) {
+      const int n = lane + 64 * t;
+      if (n < NQ2) {   // (own second layer + neighbour's) - own; 0 without a neighbour (fusedFDM.c:47-104)
+        const float own = X[face_at(f, n % NQ, n / NQ, 2)];
+        X[face_at(f, n % NQ, n / NQ, 0)] = (own + nb[f][t]) - own;
+      }
+    }
+  wave_lds_sync();
+
+  // ---- six contractions (fusedFDM.c:121-175); rows past the box repeat the last one
+  int ro[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int r = min(16 * t + c, NL * NL - 1);
+    ro[t] = (r / NL) * PS + (r % NL) * NL + KS * g;
+  }
+  fdm_f4 D[NT];
+  auto contract = [&](const float (&b)[KS], auto &&scale) {
+    float a[NT][KS];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) a[t][s] = X[ro[t] + s];
+    scale(a);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) D[t] = fdm_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) D[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][s], b[s], D[t], 0, 0, 0);
+  };
+  auto as_is = [](float (&)[NT][KS]) {};
+  // T3[p][n][m] *= invL as the next contraction reads it (KS values a row and
+  // lane against four where the sums come out).  1 / d in FP64: the hardware's
+  // estimate and one Newton step (error below 1e-13), rounded once to FP32.
+  auto by_invL = [&](float (&a)[NT][KS]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const double l = lyz[min(16 * t + c, NL * NL - 1)];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const double dg = lx[s] + l;
+        const double d = helm.x * dg + helm.y;
+        const double r0 = __builtin_amdgcn_rcp(d);
+        const double r1 = __builtin_fma(r0, __builtin_fma(-d, r0, 1.0), r0);
+        a[t][s] *= (dg > 1e-5) ? (float)r1 : 0.f;
+      }
+    }
+  };
+  auto store = [&]() {
+    wave_lds_sync();
+    if (c < NL) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) *reinterpret_cast<fdm_f4 *>(X + c * PS + 16 * t + 4 * g) = D[t];
+    }
+    wave_lds_sync();
+  };
+  contract(bf[0], as_is); store();        // T1[m][k][j]
+  contract(bf[1], as_is); store();        // T2[n][m][k]
+  contract(bf[2], as_is); store();        // T3[p][n][m]
+  contract(bb[0], by_invL); store();      // T4[i][p][n]
+  contract(bb[1], as_is); store();        // T5[j][i][p]
+  contract(bb[2], as_is); store();        // out[k][j][i]
+
+  // ---- restricted result (RAS: masked nodes, in no gather-scatter row, as zero) and overlap layers
+  float *oe = out + (int64_t)e * NP;
+  constexpr int NW = (NP + 31) / 32;
+  const uint32_t *mb = (!ASM && mbits) ? mbits + (int64_t)e * NW : nullptr;
+#pragma unroll
+  for (int t = 0; t < RI; ++t) {
+    const unsigned n = lane + 64 * t;
+    if (n < NP) {
+      float v = X[at(n / NQ2 + 1, (n / NQ) % NQ + 1, n % NQ + 1)];
+      if (mb) {   // the two mask words of these 64 nodes, by scalar loads
+        const uint32_t w0 = mb[2 * t], w1 = mb[2 * t + 1 < NW ? 2 * t + 1 : 2 * t];
+        if (((lane < 32 ? w0 : w1) >> (lane & 31)) & 1u) v = 0.f;
+      }
+      oe[n] = v;
+    }
+  }
+  if constexpr (ASM) {
+    float *ge = gout + (int64_t)e * 6 * NQ2;
+#pragma unroll
+    for (int f = 0; f < 6; ++f)
+#pragma unroll
+      for (int t = 0; t < RG; ++t) {
+        const int n = lane + 64 * t;
+        if (n < NQ2) ge[f * NQ2 + n] = X[face_at(f, n % NQ, n / NQ, 0)];
+      }
+  }
+}
+
 // epw: elements per wavefront (the tuned variant; about four by default, so
 // the prefetch has something to overlap)
 template <int NQ, int FMT>
@@ -1008,12 +1213,21 @@ template <typename T, int NQ>
 void launch_fdm_nq(bool ras, int E, const T *u, const T *S, const double *lam, double2 helm, const int4 *gmap,
                    T *out, T *gout, const uint32_t *mbits, hipStream_t s)
 {
-  using C = FdmCfg<NQ>;
-  const unsigned grid = (unsigned)((E + C::EPB - 1) / C::EPB);
-  if (ras)
-    fdm_kernel<T, NQ, false><<<grid, C::BLOCK, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
-  else
-    fdm_kernel<T, NQ, true><<<grid, C::BLOCK, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
+  if constexpr (std::is_same<T, float>::value) {
+    constexpr int W = FdmF32Cfg<NQ>::WAVES;
+    const unsigned grid = (unsigned)((E + W - 1) / W);
+    if (ras)
+      fdm_f32_kernel<NQ, false><<<grid, 64 * W, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
+    else
+      fdm_f32_kernel<NQ, true><<<grid, 64 * W, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
+  } else {
+    using C = FdmCfg<NQ>;
+    const unsigned grid = (unsigned)((E + C::EPB - 1) / C::EPB);
+    if (ras)
+      fdm_kernel<T, NQ, false><<<grid, C::BLOCK, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
+    else
+      fdm_kernel<T, NQ, true><<<grid, C::BLOCK, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
+  }
   NRS_LAUNCH_CHECK();
 }
 

@@ -216,3 +216,28 @@ def test_mg_mfma_fcg_vs_oracle(gpu, torch_mod, orc, fmt):
     assert st["converged"]
     assert abs(st["iterations"] - info["iterations"]) <= 1
     assert rel(x.cpu().numpy(), xo) <= 1e-8
+
+
+@pytest.mark.parametrize("S", ["asm", "ras"])
+@pytest.mark.parametrize("N", [2, 3, 4, 5, 6, 7, 8, 9])
+def test_fp32_boxes_every_order(gpu, torch_mod, orc, N, S):
+    """The FP32 matrix-core box solves at every box edge (tiles of 16 rows full
+    and with remainders, one to three contraction steps), 18 elements (a last
+    block of two), against the oracle's FP64 smoother.  Six sums of at most
+    N + 3 <= 12 products: 6 * 12 * 2^-24 = 4.3e-6 of the largest term, which
+    exceeds the result by less than 4 here; 2e-5 as for the other FP32 levels."""
+    torch = torch_mod
+    eg, eo, om = pair(gpu, orc, (3, 2, 3), N, [N, 1], "opt4", S)
+    import oracle.mg as omg
+    ref_mg = omg.MG(orc.BoxMesh(3, 2, 3, N, "kershaw", 0.3), [N, 1], T=np.float64, degree=3, cheby="opt4", S=S)
+    L = ref_mg.levels[0]
+    x = np.random.default_rng(N).uniform(-1, 1, L.E * L.Np)
+    x[L.el.maskIds] = 0
+    x = L.el.ogs.gs(x, "add").astype(np.float32)
+    ref = L.schwarz.apply(x.astype(np.float64))
+    out = torch.zeros(L.E * L.Np, dtype=torch.float32, device="cuda")
+    eg.mg_smoother(0, dev(torch, x), out)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert rel(got, ref) < 2e-5, rel(got, ref)
+    assert np.all(got[L.el.maskIds] == 0)
