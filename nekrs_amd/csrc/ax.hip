@@ -3,13 +3,14 @@
 //
 // Design (one element = one (N+1)^2 slab of lanes, N=7: exactly one wave64):
 //   * lane (i,j) keeps the k-pencil q(i,j,0..N) and the output pencil Aq(i,j,:)
-//     in registers, so the t-direction contractions never touch LDS;
+//     in registers (the planes are unrolled), so the t-direction contractions
+//     never touch LDS;
 //   * the r/s contractions of plane k read the plane from LDS (one 8x8 slab
 //     of doubles = 512 B), D rows/columns live in registers;
 //   * ggeo streams as 6 coalesced runs of (N+1)^2 values per plane;
 //   * the Dirichlet mask is fused into the store epilogue via a per-element
 //     bit mask (Np bits), so the operator needs no separate mask launch.
-// Small orders pack several elements per block so that a block is >= 64 lanes.
+// The other orders pack several elements per block so that whole waves are filled.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "trilin.hpp"
@@ -48,11 +49,34 @@ template <int NQ> __device__ __forceinline__ void plane_sync()
   }
 }
 
+// Elements per block of a launch variant (1, 2, 4): whole elements that fill the
+// lanes of the block's waves.  An element of NQ^2 threads leaves lanes idle at
+// most orders: order 5 ran 72 threads in two waves (56 %), order 9 100 in two
+// (78 %); the first entry of every order fills at least 94 %.  Larger blocks than
+// these would cap the registers of the high orders.  Order 7 is one element per
+// wave.
 template <int NQ, int MULT = 1> struct AxShape {
-  // elements per block: fill at least one wave64, times the tuned multiplier
-  static constexpr int NE = ((NQ * NQ >= 64) ? 1 : (64 + NQ * NQ - 1) / (NQ * NQ)) * MULT;
+  static constexpr int ne()
+  {
+    switch (NQ) {
+      case 2: return 16 * MULT;                                 // 64, 128, 256 threads
+      case 3: return 7 * MULT;                                  // 63, 126, 252
+      case 4: return 4 * MULT;                                  // 64, 128, 256
+      case 5: return 5 * MULT;                                  // 125, 250, 500
+      case 6: return MULT == 1 ? 7 : MULT == 2 ? 14 : 5;        // 252, 504, 180
+      case 7: return MULT == 1 ? 5 : MULT == 2 ? 13 : 9;        // 245, 637, 441
+      case 9: return MULT == 1 ? 3 : MULT == 2 ? 6 : 7;         // 243, 486, 567
+      case 10: return MULT == 1 ? 5 : MULT == 2 ? 2 : 1;        // 500, 200, 100
+      default: return MULT;                                     // order 7: 64, 128, 256
+    }
+  }
+  static constexpr int NE = ne();
   static constexpr int THREADS = NQ * NQ * NE;
 };
+
+// Where the geometric factors come from: streamed one plane ahead, streamed
+// all planes at once, or formed from the element corners.
+enum { GEO_STREAM = 0, GEO_AHEAD = 1, GEO_CORNERS = 2 };
 
 // -------------------------------------------------------------------------------------
 // Single-field apply.  Restates ellipticPartialAxCoeffHex3D
@@ -60,6 +84,13 @@ template <int NQ, int MULT = 1> struct AxShape {
 //   qr = sum_m D[i][m] q(m,j,k), qs = sum_m D[j][m] q(i,m,k), qt = sum_m D[k][m] q(i,j,m)
 //   [Gqr,Gqs,Gqt] = lambda0 * G * [qr,qs,qt]
 //   Aq = sum_m D[m][i] Gqr(m,j,k) + D[m][j] Gqs(i,m,k) + D[m][k] Gqt(i,j,m) (+ GwJ lambda1 q)
+// The planes are unrolled, so the pencils are indexed at compile time (a rolled
+// loop selected q(k) and the row of Aq with a compare per entry: 30 of about 190
+// vector instructions a plane in FP64); the scheduling barrier keeps a plane's
+// loads from being hoisted over the planes before it, which would cost the
+// registers of every plane's factors.  HBM-bound at size: FP64, order 7, 32^3
+// elements with the face fusion 210 us rolled, 178 us (1.074 GB, 6.0 TB/s);
+// Helmholtz, order 9, 6840 elements 156 us, 92 us with the packing of AxShape.
 // -------------------------------------------------------------------------------------
 //
 // FUSEX: the block's consecutive elements e, e+1 with fx[e] = 1 share their
@@ -67,11 +98,16 @@ template <int NQ, int MULT = 1> struct AxShape {
 // here through LDS (both copies get v_e + v_e+1, the gather-scatter's pair sum,
 // bit for bit) and the caller's gather-scatter handle leaves them out.
 //
-// TRI: trilinear elements.  The geometric factors are not read but formed at
-// each node from the element's eight corners (corners [E][3][8]) and the GLL
-// nodes and weights (zw [2][NQ]) by TriGeo (trilin.hpp).
-template <typename T, int NQ, int MULT, bool POISSON, bool LFIELD, bool FUSEX = false, bool TRI = false>
-__global__ void __launch_bounds__((AxShape<NQ, MULT>::THREADS), AX_WAVES_PER_EU)
+// GEO_AHEAD: every plane's factors in flight before the first plane, for a mesh
+// of so few elements that a wave has a SIMD to itself and waits out each
+// plane's memory latency otherwise.
+//
+// GEO_CORNERS: trilinear elements.  The geometric factors are not read but
+// formed at each node from the element's eight corners (corners [E][3][8]) and
+// the GLL nodes and weights (zw [2][NQ]) by TriGeo (trilin.hpp).
+template <typename T, int NQ, int MULT, bool POISSON, bool LFIELD, bool FUSEX = false, int GEO = GEO_STREAM>
+__global__ void __launch_bounds__((AxShape<NQ, MULT>::THREADS),
+                                  (GEO == GEO_AHEAD ? 1 : (sizeof(T) == 8 && NQ >= 9) ? 2 : AX_WAVES_PER_EU))
 ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
           const T *__restrict__ Dg, const T *__restrict__ lam0, const T *__restrict__ lam1,
           const T *__restrict__ q, T *__restrict__ Aq, const uint32_t *__restrict__ maskBits,
@@ -79,7 +115,7 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
           const T *__restrict__ zw = nullptr)
 {
   constexpr int NE = AxShape<NQ, MULT>::NE;
-  constexpr int NP = NQ * NQ * NQ;
+  constexpr int NP = NQ * NQ * NQ, NQ2 = NQ * NQ;
   constexpr int NW = (NP + 31) / 32;
   __shared__ T s_D[NQ][NQ];
   __shared__ T s_q[NE][NQ][NQ];
@@ -89,15 +125,37 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
   const int t = threadIdx.x;
   const int i = t % NQ;
   const int j = (t / NQ) % NQ;
-  const int le = (NE == 1) ? 0 : t / (NQ * NQ);
+  const int le = (NE == 1) ? 0 : t / NQ2;
   const int eidx = blockIdx.x * NE + le;
   const bool active = eidx < E;
   int64_t e = active ? (elist ? elist[eidx] : eidx) : 0;
-  if (NE == 1 || NQ * NQ == 64) e = __builtin_amdgcn_readfirstlane((int)e);   // wave-uniform element
+  if (NQ2 == 64) e = __builtin_amdgcn_readfirstlane((int)e);   // wave-uniform element
 
-  if (t < NQ * NQ) s_D[t / NQ][t % NQ] = Dg[t];
+  const int lid = j * NQ + i;          // lane offset inside a plane (32-bit)
+  const T *qe = q + e * NP;
+  const T *G = ggeo + e * 7 * NP;
+  constexpr int NG = POISSON ? 6 : 7;
+  constexpr int NA = (GEO == GEO_AHEAD) ? NQ : 2;   // planes of factors held
+  T g[NA][7];
+#define NRS_LOAD_G(k_, p_)                                                                            \
+  do {                                                                                              \
+    _Pragma("unroll") for (int c = 0; c < NG; ++c) g[p_][c] = stream_load(G + c * NP + (k_) * NQ2 + lid); \
+  } while (0)
+  T r_q[NQ], r_Aq[NQ];
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    r_q[k] = qe[k * NQ2 + lid];
+    r_Aq[k] = T(0);
+  }
+  if constexpr (GEO == GEO_AHEAD) {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) NRS_LOAD_G(k, k);
+  } else if constexpr (GEO == GEO_STREAM) {
+    NRS_LOAD_G(0, 0);
+  }
+
+  if (t < NQ2) s_D[t / NQ][t % NQ] = Dg[t];
   __syncthreads();
-
   T Di[NQ], Dj[NQ], DTi[NQ], DTj[NQ];
 #pragma unroll
   for (int m = 0; m < NQ; ++m) {
@@ -107,64 +165,35 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
     DTj[m] = s_D[m][j];
   }
 
-  const int lid = j * NQ + i;          // lane offset inside a plane (32-bit)
-  const T *qe = q + e * NP;
-  const T *G = ggeo + e * 7 * NP;
-  T r_q[NQ], r_Aq[NQ];
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    r_q[k] = active ? qe[k * NQ * NQ + lid] : T(0);
-    r_Aq[k] = T(0);
-  }
-
   const T l0c = LFIELD ? T(0) : lam0[0];
   const T l1c = (LFIELD || POISSON) ? T(0) : lam1[0];
 
-  // geometric factors of plane 0; later planes are prefetched one plane ahead
-  // (TRI: the corner differences that the derivatives of the map take at this
-  // lane's (r, s), formed once per element)
-  T g[7];
+  // corners: what the derivatives of the map take at this lane's (r, s), once per element
   TriGeo<T> tri;
-  if constexpr (TRI) {
-    tri.init(corners + e * 24, zw[i], zw[j], zw[NQ + i], zw[NQ + j]);
-  } else {
-#pragma unroll
-    for (int c = 0; c < 7; ++c) g[c] = (active && (c < 6 || !POISSON)) ? stream_load(G + c * NP + lid) : T(0);
-  }
+  if constexpr (GEO == GEO_CORNERS) tri.init(corners + e * 24, zw[i], zw[j], zw[NQ + i], zw[NQ + j]);
 
-#pragma unroll 1
+#pragma unroll
   for (int k = 0; k < NQ; ++k) {
-    const int n = k * NQ * NQ;
-    T qk = r_q[0];
-#pragma unroll
-    for (int m = 1; m < NQ; ++m) qk = (k == m) ? r_q[m] : qk;
-    T gn[7];
-    if constexpr (TRI) {
-      T v[10];
-      tri.at(zw[k], zw[NQ + k], v);
-      const T rx = v[0], ry = v[1], rz = v[2], sx = v[3], sy = v[4], sz = v[5], tx = v[6], ty = v[7], tz = v[8];
-      const T JW = v[9];
-      g[kG00] = JW * (rx * rx + ry * ry + rz * rz);
-      g[kG01] = JW * (rx * sx + ry * sy + rz * sz);
-      g[kG02] = JW * (rx * tx + ry * ty + rz * tz);
-      g[kG11] = JW * (sx * sx + sy * sy + sz * sz);
-      g[kG12] = JW * (sx * tx + sy * ty + sz * tz);
-      g[kG22] = JW * (tx * tx + ty * ty + tz * tz);
-      g[kGWJ] = JW;
-    } else {
-      const bool more = active && (k + 1 < NQ);
-#pragma unroll
-      for (int c = 0; c < 7; ++c)
-        gn[c] = (more && (c < 6 || !POISSON)) ? stream_load(G + c * NP + n + NQ * NQ + lid) : T(0);
+    const int n = k * NQ2;
+    if constexpr (GEO != GEO_AHEAD) __builtin_amdgcn_sched_barrier(0);
+    const int p = (GEO == GEO_AHEAD) ? k : k & 1;
+    if constexpr (GEO == GEO_STREAM) {
+      if (k + 1 < NQ) NRS_LOAD_G(k + 1, 1 - p);
+    } else if constexpr (GEO == GEO_CORNERS) {
+      T v[7];
+      tri.metric(zw[k], zw[NQ + k], v);
+      g[p][kG00] = v[0]; g[p][kG01] = v[1]; g[p][kG02] = v[2];
+      g[p][kG11] = v[3]; g[p][kG12] = v[4]; g[p][kG22] = v[5];
+      g[p][kGWJ] = v[6];
     }
     T l0 = l0c, l1 = l1c;
-    if (LFIELD && active) {
+    if (LFIELD) {
       l0 = lam0[e * NP + n + lid];
       if (!POISSON) l1 = lam1[e * NP + n + lid];
     }
-    const T G00 = g[kG00], G01 = g[kG01], G02 = g[kG02], G11 = g[kG11], G12 = g[kG12], G22 = g[kG22];
+    const T G00 = g[p][kG00], G01 = g[p][kG01], G02 = g[p][kG02], G11 = g[p][kG11], G12 = g[p][kG12], G22 = g[p][kG22];
 
-    s_q[le][j][i] = qk;
+    s_q[le][j][i] = r_q[k];
     T qt = 0;
 #pragma unroll
     for (int m = 0; m < NQ; ++m) qt += Dg[k * NQ + m] * r_q[m];
@@ -191,15 +220,14 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
 #pragma unroll
     for (int m = 0; m < NQ; ++m) b += DTj[m] * s_Gs[le][m][i];
     T ab = a + b;
-    if (!POISSON) ab += g[kGWJ] * l1 * qk;
+    if (!POISSON) ab += g[p][kGWJ] * l1 * r_q[k];
 #pragma unroll
     for (int m = 0; m < NQ; ++m) r_Aq[m] += Dg[k * NQ + m] * Gqt;
+    r_Aq[k] += ab;
+    // the sums are needed only at the end: without this the compiler keeps every
+    // plane's operands in registers and adds them up there
 #pragma unroll
-    for (int m = 0; m < NQ; ++m) r_Aq[m] += (k == m) ? ab : T(0);
-    if constexpr (!TRI) {
-#pragma unroll
-      for (int c = 0; c < 7; ++c) g[c] = gn[c];
-    }
+    for (int m = 0; m < NQ; ++m) asm volatile("" : "+v"(r_Aq[m]));
   }
 
   if constexpr (FUSEX) {
@@ -228,14 +256,24 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
     const uint32_t *mb = maskBits + e * NW;
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-      const int n = k * NQ * NQ + j * NQ + i;
+      const int n = k * NQ2 + lid;
       const bool masked = (mb[n >> 5] >> (n & 31)) & 1u;
-      Ae[k * NQ * NQ] = masked ? T(0) : r_Aq[k];
+      Ae[k * NQ2] = masked ? T(0) : r_Aq[k];
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) Ae[k * NQ * NQ] = r_Aq[k];
+    for (int k = 0; k < NQ; ++k) Ae[k * NQ2] = r_Aq[k];
   }
+}
+
+// All planes' factors at once where the launch has at most one wave per SIMD
+// (1024 on the chip): latency is what such a launch waits for (FP64, order 7, 64
+// elements: 10.1 us one plane ahead, 6.1 us; 512 elements 12.8 and 10.7 us); with
+// more waves per SIMD they hide each other's, and the registers would halve
+// their number.  FP64 above order 7 would spill.
+template <typename T, int NQ, int MULT> static bool ax_ahead(int E)
+{
+  return (sizeof(T) == 4 || NQ <= 8) && (int64_t)E * NQ * NQ <= 64 * 1024;
 }
 
 template <typename T, int NQ, int MULT>
@@ -246,6 +284,18 @@ static void launch_ax_nqm(int E, const int *elist, const T *ggeo, const T *D, co
   using S = AxShape<NQ, MULT>;
   const unsigned grid = (unsigned)((E + S::NE - 1) / S::NE);
   if (grid == 0) return;
+  if constexpr (sizeof(T) == 4 || NQ <= 8) {
+    if (ax_ahead<T, NQ, MULT>(E) && !lfield) {
+      if (poisson)
+        ax_kernel<T, NQ, MULT, true, false, false, GEO_AHEAD><<<grid, S::THREADS, 0, s>>>(E, elist, ggeo, D, l0, l1, q,
+                                                                                          Aq, maskBits);
+      else
+        ax_kernel<T, NQ, MULT, false, false, false, GEO_AHEAD><<<grid, S::THREADS, 0, s>>>(E, elist, ggeo, D, l0, l1,
+                                                                                           q, Aq, maskBits);
+      NRS_LAUNCH_CHECK();
+      return;
+    }
+  }
   if (poisson && !lfield)
     ax_kernel<T, NQ, MULT, true, false><<<grid, S::THREADS, 0, s>>>(E, elist, ggeo, D, l0, l1, q, Aq, maskBits);
   else if (poisson && lfield)
@@ -297,10 +347,10 @@ static void launch_ax_trilin_nq(int mult, int E, const T *corners, const T *zw, 
     const unsigned grid = (unsigned)((E + S::NE - 1) / S::NE);                                       \
     if (grid == 0) return;                                                                           \
     if (poisson)                                                                                     \
-      ax_kernel<T, NQ, M_, true, false, false, true><<<grid, S::THREADS, 0, s>>>(                     \
+      ax_kernel<T, NQ, M_, true, false, false, GEO_CORNERS><<<grid, S::THREADS, 0, s>>>(              \
           E, nullptr, nullptr, D, l0, l1, q, Aq, maskBits, nullptr, corners, zw);                    \
     else                                                                                             \
-      ax_kernel<T, NQ, M_, false, false, false, true><<<grid, S::THREADS, 0, s>>>(                    \
+      ax_kernel<T, NQ, M_, false, false, false, GEO_CORNERS><<<grid, S::THREADS, 0, s>>>(             \
           E, nullptr, nullptr, D, l0, l1, q, Aq, maskBits, nullptr, corners, zw);                    \
   }
   switch (mult) {
@@ -342,6 +392,16 @@ static void launch_ax_fused_m(int E, const T *ggeo, const T *D, const T *l0, con
   static_assert(S::NE == M, "one element per wave at N = 7");
   const unsigned grid = (unsigned)((E + S::NE - 1) / S::NE);
   if (grid == 0) return;
+  if (ax_ahead<T, 8, M>(E)) {
+    if (poisson)
+      ax_kernel<T, 8, M, true, false, true, GEO_AHEAD><<<grid, S::THREADS, 0, s>>>(E, nullptr, ggeo, D, l0, l1, q, Aq,
+                                                                                   maskBits, fx);
+    else
+      ax_kernel<T, 8, M, false, false, true, GEO_AHEAD><<<grid, S::THREADS, 0, s>>>(E, nullptr, ggeo, D, l0, l1, q, Aq,
+                                                                                    maskBits, fx);
+    NRS_LAUNCH_CHECK();
+    return;
+  }
   if (poisson)
     ax_kernel<T, 8, M, true, false, true><<<grid, S::THREADS, 0, s>>>(E, nullptr, ggeo, D, l0, l1, q, Aq,
                                                                       maskBits, fx);

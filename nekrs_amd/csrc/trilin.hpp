@@ -34,6 +34,28 @@ template <typename T> struct TriGeo {
     }
   }
 
+  // G00 G01 G02 G11 G12 G22 GWJ at the plane t: with the cofactors c (J grad r and
+  // so on, not divided by J), G_ab = (w / J) c_a . c_b
+  __device__ __forceinline__ void metric(T t, T wk, T (&v)[7]) const
+  {
+    const T ht0 = T(0.5) * (T(1) - t), ht1 = T(0.5) * (T(1) + t);
+    const T xr = ht0 * dRB[0] + ht1 * dRT[0], yr = ht0 * dRB[1] + ht1 * dRT[1], zr = ht0 * dRB[2] + ht1 * dRT[2];
+    const T xs = ht0 * dSB[0] + ht1 * dST[0], ys = ht0 * dSB[1] + ht1 * dST[1], zs = ht0 * dSB[2] + ht1 * dST[2];
+    const T xt = dT[0], yt = dT[1], zt = dT[2];
+    const T rx = ys * zt - zs * yt, ry = zs * xt - xs * zt, rz = xs * yt - ys * xt;
+    const T sx = zr * yt - yr * zt, sy = xr * zt - zr * xt, sz = yr * xt - xr * yt;
+    const T tx = yr * zs - zr * ys, ty = zr * xs - xr * zs, tz = xr * ys - yr * xs;
+    const T J = xr * rx + yr * ry + zr * rz;
+    const T w = wij * wk, f = w / J;
+    v[0] = f * (rx * rx + ry * ry + rz * rz);
+    v[1] = f * (rx * sx + ry * sy + rz * sz);
+    v[2] = f * (rx * tx + ry * ty + rz * tz);
+    v[3] = f * (sx * sx + sy * sy + sz * sz);
+    v[4] = f * (sx * tx + sy * ty + sz * tz);
+    v[5] = f * (tx * tx + ty * ty + tz * tz);
+    v[6] = J * w;
+  }
+
   // g = rx ry rz sx sy sz tx ty tz JW at the plane t (GLL weight wk)
   __device__ __forceinline__ void at(T t, T wk, T (&g)[10]) const
   {
