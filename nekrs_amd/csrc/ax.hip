@@ -104,7 +104,7 @@ enum { GEO_STREAM = 0, GEO_AHEAD = 1, GEO_CORNERS = 2 };
 //
 // GEO_CORNERS: trilinear elements.  The geometric factors are not read but
 // formed at each node from the element's eight corners (corners [E][3][8]) and
-// the GLL nodes and weights (zw [2][NQ]) by TriGeo (trilin.hpp).
+// the GLL nodes and weights (zw [2][NQ]) by TriMetric (trilin.hpp).
 template <typename T, int NQ, int MULT, bool POISSON, bool LFIELD, bool FUSEX = false, int GEO = GEO_STREAM>
 __global__ void __launch_bounds__((AxShape<NQ, MULT>::THREADS),
                                   (GEO == GEO_AHEAD ? 1 : (sizeof(T) == 8 && NQ >= 9) ? 2 : AX_WAVES_PER_EU))
@@ -169,7 +169,7 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
   const T l1c = (LFIELD || POISSON) ? T(0) : lam1[0];
 
   // corners: what the derivatives of the map take at this lane's (r, s), once per element
-  TriGeo<T> tri;
+  TriMetric<T> tri;
   if constexpr (GEO == GEO_CORNERS) tri.init(corners + e * 24, zw[i], zw[j], zw[NQ + i], zw[NQ + j]);
 
 #pragma unroll
@@ -179,20 +179,12 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
     const int p = (GEO == GEO_AHEAD) ? k : k & 1;
     if constexpr (GEO == GEO_STREAM) {
       if (k + 1 < NQ) NRS_LOAD_G(k + 1, 1 - p);
-    } else if constexpr (GEO == GEO_CORNERS) {
-      T v[7];
-      tri.metric(zw[k], zw[NQ + k], v);
-      g[p][kG00] = v[0]; g[p][kG01] = v[1]; g[p][kG02] = v[2];
-      g[p][kG11] = v[3]; g[p][kG12] = v[4]; g[p][kG22] = v[5];
-      g[p][kGWJ] = v[6];
     }
     T l0 = l0c, l1 = l1c;
     if (LFIELD) {
       l0 = lam0[e * NP + n + lid];
       if (!POISSON) l1 = lam1[e * NP + n + lid];
     }
-    const T G00 = g[p][kG00], G01 = g[p][kG01], G02 = g[p][kG02], G11 = g[p][kG11], G12 = g[p][kG12], G22 = g[p][kG22];
-
     s_q[le][j][i] = r_q[k];
     T qt = 0;
 #pragma unroll
@@ -205,12 +197,31 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
       qr += Di[m] * s_q[le][j][m];
       qs += Dj[m] * s_q[le][m][i];
     }
-    T Gqr = G00 * qr; Gqr += G01 * qs; Gqr += G02 * qt;
-    T Gqs = G01 * qr; Gqs += G11 * qs; Gqs += G12 * qt;
-    T Gqt = G02 * qr; Gqt += G12 * qs; Gqt += G22 * qt;
-    s_Gr[le][j][i] = l0 * Gqr;
-    s_Gs[le][j][i] = l0 * Gqs;
-    Gqt *= l0;
+    T Gqr, Gqs, Gqt, gwj;
+    if constexpr (GEO == GEO_CORNERS) {
+      T c[9], f;
+      tri.at(zw[k], zw[NQ + k], c, f, gwj);
+      f *= l0;
+      T v[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        v[d] = c[d] * qr; v[d] += c[3 + d] * qs; v[d] += c[6 + d] * qt;
+        v[d] *= f;
+      }
+      Gqr = c[0] * v[0]; Gqr += c[1] * v[1]; Gqr += c[2] * v[2];
+      Gqs = c[3] * v[0]; Gqs += c[4] * v[1]; Gqs += c[5] * v[2];
+      Gqt = c[6] * v[0]; Gqt += c[7] * v[1]; Gqt += c[8] * v[2];
+    } else {
+      const T G00 = g[p][kG00], G01 = g[p][kG01], G02 = g[p][kG02];
+      const T G11 = g[p][kG11], G12 = g[p][kG12], G22 = g[p][kG22];
+      Gqr = G00 * qr; Gqr += G01 * qs; Gqr += G02 * qt;
+      Gqs = G01 * qr; Gqs += G11 * qs; Gqs += G12 * qt;
+      Gqt = G02 * qr; Gqt += G12 * qs; Gqt += G22 * qt;
+      Gqr *= l0; Gqs *= l0; Gqt *= l0;
+      gwj = POISSON ? T(0) : g[p][kGWJ];
+    }
+    s_Gr[le][j][i] = Gqr;
+    s_Gs[le][j][i] = Gqs;
     plane_sync<NQ>();
 
     T a = 0;
@@ -220,7 +231,7 @@ ax_kernel(int E, const int *__restrict__ elist, const T *__restrict__ ggeo,
 #pragma unroll
     for (int m = 0; m < NQ; ++m) b += DTj[m] * s_Gs[le][m][i];
     T ab = a + b;
-    if (!POISSON) ab += g[p][kGWJ] * l1 * r_q[k];
+    if (!POISSON) ab += gwj * l1 * r_q[k];
 #pragma unroll
     for (int m = 0; m < NQ; ++m) r_Aq[m] += Dg[k * NQ + m] * Gqt;
     r_Aq[k] += ab;
