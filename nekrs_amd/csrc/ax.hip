@@ -471,125 +471,151 @@ template void launch_ax<float>(int, int, const int *, const float *, const float
 // the geometric factors are read once for the three fields.
 // -------------------------------------------------------------------------------------
 // Same scheme as ax_kernel: one (i,j) column per lane, the k-pencils of q and
-// of the result in registers with the k loop rolled (static register
-// indexing through selects), r/s contractions through LDS slabs, geometric
-// factors prefetched one plane ahead and shared by the three fields.
+// of the result in registers over unrolled planes, r/s contractions through LDS slabs, geometric factors prefetched one
+// plane ahead and shared by the three fields, blocks of whole elements that fill
+// their waves (AxShape), the Dirichlet mask in the store (maskBits, optional).
+// HBM-bound in the count of bytes, held back by two waves per SIMD (registers):
+// order 5, 5814 curved elements 57.8 -> 33 us (131 MB, 3.9 TB/s), and no mask pass.
+// coefficient fields at order 9: smaller blocks, for the registers
+template <int NQ, bool LFIELD> using BlockAxShape = AxShape<NQ, (NQ == 10 && LFIELD) ? 2 : 1>;
 template <int NQ, bool LFIELD>
-__global__ void __launch_bounds__(AxShape<NQ>::THREADS, LFIELD ? 1 : 2)
+__global__ void __launch_bounds__((BlockAxShape<NQ, LFIELD>::THREADS), LFIELD ? 1 : 2)
 block_ax_kernel(int E, int64_t offset, int64_t loffset, const double *__restrict__ ggeo,
                 const double *__restrict__ Dg, const double *__restrict__ lam0,
                 const double *__restrict__ lam1, const double *__restrict__ q,
-                double *__restrict__ Aq)
+                double *__restrict__ Aq, const uint32_t *__restrict__ maskBits)
 {
-  constexpr int NE = AxShape<NQ>::NE;
-  constexpr int NP = NQ * NQ * NQ;
+  constexpr int NE = BlockAxShape<NQ, LFIELD>::NE;
+  constexpr int NP = NQ * NQ * NQ, NQ2 = NQ * NQ;
+  constexpr int NW = (NP + 31) / 32;
   constexpr int NF = 3;
   __shared__ double s_D[NQ][NQ];
   __shared__ double s_q[NF][NE][NQ][NQ];
   __shared__ double s_Gr[NF][NE][NQ][NQ];
   __shared__ double s_Gs[NF][NE][NQ][NQ];
   const int t = threadIdx.x;
-  const int i = t % NQ, j = (t / NQ) % NQ, le = t / (NQ * NQ);
+  const int i = t % NQ, j = (t / NQ) % NQ, le = t / NQ2;
   const int eidx = blockIdx.x * NE + le;
-  const bool active = eidx < E;
+  const bool active = eidx < E;      // inactive lanes read element 0 and store nothing
   const int64_t e = active ? eidx : 0;
-  if (t < NQ * NQ) s_D[t / NQ][t % NQ] = Dg[t];
-  __syncthreads();
   const int lid = j * NQ + i;
   double r_q[NF][NQ], r_Aq[NF][NQ];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-      r_q[f][k] = active ? q[f * offset + e * NP + k * NQ * NQ + lid] : 0.0;
+      r_q[f][k] = q[f * offset + e * NP + k * NQ2 + lid];
       r_Aq[f][k] = 0.0;
     }
   const double *G = ggeo + e * 7 * NP + lid;
-  double g[7];
+  double g[2][7];
 #pragma unroll
-  for (int c = 0; c < 7; ++c) g[c] = active ? stream_load(G + c * NP) : 0.0;
+  for (int c = 0; c < 7; ++c) g[0][c] = stream_load(G + c * NP);
+  if (t < NQ2) s_D[t / NQ][t % NQ] = Dg[t];
+  __syncthreads();
+  // D rows and columns in registers up to order 7; above, they would spill and
+  // are read from LDS, once a plane for the three fields
+  constexpr bool DREG = NQ <= 8;
+  double Di[NQ], Dj[NQ], DTi[NQ], DTj[NQ];
+  auto rows = [&]() {
+#pragma unroll
+    for (int m = 0; m < NQ; ++m) { Di[m] = s_D[i][m]; Dj[m] = s_D[j][m]; }
+  };
+  auto cols = [&]() {
+#pragma unroll
+    for (int m = 0; m < NQ; ++m) { DTi[m] = s_D[m][i]; DTj[m] = s_D[m][j]; }
+  };
+  if (DREG) { rows(); cols(); }
   const double l0c = LFIELD ? 0.0 : lam0[0];
   const double l1c = LFIELD ? 0.0 : lam1[0];
 
-#pragma unroll 1
-  for (int k = 0; k < NQ; ++k) {
-    const int n = k * NQ * NQ;
-    const int64_t id = e * NP + n + lid;
-    double gn[7];
-    const bool more = active && (k + 1 < NQ);
 #pragma unroll
-    for (int c = 0; c < 7; ++c) gn[c] = more ? stream_load(G + c * NP + n + NQ * NQ) : 0.0;
-    double qk[NF], qt[NF];
+  for (int k = 0; k < NQ; ++k) {
+    __builtin_amdgcn_sched_barrier(0);   // as in ax_kernel
+    const int64_t id = e * NP + k * NQ2 + lid;
+    const int p = k & 1;
+    if (k + 1 < NQ) {
+#pragma unroll
+      for (int c = 0; c < 7; ++c) g[1 - p][c] = stream_load(G + c * NP + (k + 1) * NQ2);
+    }
+    double qt[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      qk[f] = r_q[f][0];
-#pragma unroll
-      for (int m = 1; m < NQ; ++m) qk[f] = (k == m) ? r_q[f][m] : qk[f];
-      s_q[f][le][j][i] = qk[f];
+      s_q[f][le][j][i] = r_q[f][k];
       double a = 0.0;
 #pragma unroll
-      for (int m = 0; m < NQ; ++m) a += s_D[k][m] * r_q[f][m];
+      for (int m = 0; m < NQ; ++m) a += Dg[k * NQ + m] * r_q[f][m];
       qt[f] = a;
     }
-    __syncthreads();
+    plane_sync<NQ>();
+    if (!DREG) rows();
     double Gqt[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       double qr = 0.0, qs = 0.0;
 #pragma unroll
       for (int m = 0; m < NQ; ++m) {
-        qr += s_D[i][m] * s_q[f][le][j][m];
-        qs += s_D[j][m] * s_q[f][le][m][i];
+        qr += Di[m] * s_q[f][le][j][m];
+        qs += Dj[m] * s_q[f][le][m][i];
       }
-      const double l0 = LFIELD ? (active ? lam0[f * loffset + id] : 0.0) : l0c;
-      s_Gr[f][le][j][i] = l0 * (g[kG00] * qr + g[kG01] * qs + g[kG02] * qt[f]);
-      s_Gs[f][le][j][i] = l0 * (g[kG01] * qr + g[kG11] * qs + g[kG12] * qt[f]);
-      Gqt[f] = l0 * (g[kG02] * qr + g[kG12] * qs + g[kG22] * qt[f]);
+      const double l0 = LFIELD ? lam0[f * loffset + id] : l0c;
+      s_Gr[f][le][j][i] = l0 * (g[p][kG00] * qr + g[p][kG01] * qs + g[p][kG02] * qt[f]);
+      s_Gs[f][le][j][i] = l0 * (g[p][kG01] * qr + g[p][kG11] * qs + g[p][kG12] * qt[f]);
+      Gqt[f] = l0 * (g[p][kG02] * qr + g[p][kG12] * qs + g[p][kG22] * qt[f]);
     }
-    __syncthreads();
+    plane_sync<NQ>();
+    if (!DREG) cols();
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      const double l1 = LFIELD ? (active ? lam1[f * loffset + id] : 0.0) : l1c;
+      const double l1 = LFIELD ? lam1[f * loffset + id] : l1c;
       double a = 0.0, b = 0.0;
 #pragma unroll
       for (int m = 0; m < NQ; ++m) {
-        a += s_D[m][i] * s_Gr[f][le][j][m];
-        b += s_D[m][j] * s_Gs[f][le][m][i];
+        a += DTi[m] * s_Gr[f][le][j][m];
+        b += DTj[m] * s_Gs[f][le][m][i];
       }
-      const double ab = a + b + g[kGWJ] * l1 * qk[f];
+      const double ab = a + b + g[p][kGWJ] * l1 * r_q[f][k];
 #pragma unroll
-      for (int m = 0; m < NQ; ++m) r_Aq[f][m] += s_D[k][m] * Gqt[f];
-#pragma unroll
-      for (int m = 0; m < NQ; ++m) r_Aq[f][m] += (k == m) ? ab : 0.0;
+      for (int m = 0; m < NQ; ++m) r_Aq[f][m] += Dg[k * NQ + m] * Gqt[f];
+      r_Aq[f][k] += ab;
     }
 #pragma unroll
-    for (int c = 0; c < 7; ++c) g[c] = gn[c];
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int m = 0; m < NQ; ++m) asm volatile("" : "+v"(r_Aq[f][m]));   // as in ax_kernel
   }
   if (!active) return;
+  const uint32_t *mb = maskBits ? maskBits + e * NW : nullptr;
 #pragma unroll
-  for (int f = 0; f < NF; ++f)
+  for (int k = 0; k < NQ; ++k) {
+    const int n = k * NQ2 + lid;
+    const bool masked = mb && ((mb[n >> 5] >> (n & 31)) & 1u);
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) Aq[f * offset + e * NP + k * NQ * NQ + lid] = r_Aq[f][k];
+    for (int f = 0; f < NF; ++f) Aq[f * offset + e * NP + n] = masked ? 0.0 : r_Aq[f][k];
+  }
 }
 
 void launch_block_ax(int N, int E, int64_t offset, int64_t loffset, const double *ggeo,
                      const double *D, const double *l0, const double *l1, const double *q,
-                     double *Aq, hipStream_t s, bool lfield)
+                     double *Aq, hipStream_t s, bool lfield, const uint32_t *maskBits)
 {
-#define BLK(NQ)                                                                              \
-  case NQ: {                                                                                 \
-    const unsigned g = (unsigned)((E + AxShape<NQ>::NE - 1) / AxShape<NQ>::NE);              \
-    if (g && lfield)                                                                         \
-      block_ax_kernel<NQ, true><<<g, AxShape<NQ>::THREADS, 0, s>>>(E, offset, loffset, ggeo, D, l0, l1, q, Aq); \
-    else if (g)                                                                              \
-      block_ax_kernel<NQ, false><<<g, AxShape<NQ>::THREADS, 0, s>>>(E, offset, loffset, ggeo, D, l0, l1, q, Aq); \
-    break;                                                                                   \
+#define BLK1(NQ, LF)                                                                         \
+  {                                                                                          \
+    using S = BlockAxShape<NQ, LF>;                                                          \
+    const unsigned g = (unsigned)((E + S::NE - 1) / S::NE);                                  \
+    if (g)                                                                                   \
+      block_ax_kernel<NQ, LF><<<g, S::THREADS, 0, s>>>(E, offset, loffset, ggeo, D, l0, l1, q, Aq, maskBits); \
   }
+#define BLK(NQ)                                                                              \
+  case NQ:                                                                                   \
+    if (lfield) BLK1(NQ, true) else BLK1(NQ, false)                                          \
+    break;
   switch (N + 1) {
     BLK(2) BLK(3) BLK(4) BLK(5) BLK(6) BLK(7) BLK(8) BLK(9) BLK(10)
     default: throw Error(NRS_ERR_UNSUPPORTED, "block Ax: order N must be 1..9");
   }
 #undef BLK
+#undef BLK1
   NRS_LAUNCH_CHECK();
 }
 

@@ -523,12 +523,11 @@ static void mask_fields(nrs_elliptic *el, double *v, hipStream_t s)
 void elliptic_operator(nrs_elliptic *el, const double *q, double *Aq, bool masked, hipStream_t s)
 {
   if (el->Nf > 1) {
-    // three fields: the block apply (ellipticBlockPartialAxCoeffHex3D), the
-    // mask of each field, one gather-scatter of the three vectors
+    // three fields: the block apply (ellipticBlockPartialAxCoeffHex3D) with the
+    // mask in its store, one gather-scatter of the three vectors
     // (oogs::startFinish with k = 3)
     launch_block_ax(el->N, el->E, el->Nlocal, 0, el->ggeo.get(), el->D.get(), el->l0ptr(),
-                    el->l1ptr(), q, Aq, s, el->lfield());
-    if (masked) mask_fields(el, Aq, s);
+                    el->l1ptr(), q, Aq, s, el->lfield(), masked ? el->maskBits.get() : nullptr);
     ogs_gather_scatter<double>(el->ogs, Aq, el->Nf, el->Nlocal, NRS_ADD, s);
     return;
   }

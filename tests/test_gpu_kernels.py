@@ -51,6 +51,27 @@ def test_ax_vs_oracle(gpu, torch_mod, orc, N, T, kind):
     assert rel(host(Aq), ref) < tol
 
 
+@pytest.mark.parametrize("N", [1, 2, 4, 5, 6, 7])
+@pytest.mark.parametrize("T", [np.float64, np.float32])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_ax_at_the_load_ahead_line(gpu, torch_mod, orc, N, T, extra):
+    """The launch loads every plane's factors ahead up to E (N+1)^2 = 65536 threads
+    and one plane ahead beyond: the last mesh of one form and the first of the
+    other (a last block of fewer elements in both), against the oracle with the
+    bars of test_ax_vs_oracle."""
+    torch = torch_mod
+    E = 65536 // (N + 1) ** 2 + extra
+    m = orc.BoxMesh(E, 1, 1, N, "kershaw", 0.3)
+    q = np.random.default_rng(N).uniform(-1, 1, E * m.Np)
+    ref = orc.ax(N, m.ggeo.astype(T), m.D.astype(T), q.astype(T), lambda0=1.3, lambda1=2.0, poisson=False, dtype=T)
+    Aq = torch.zeros(E * m.Np, dtype=torch.float64 if T == np.float64 else torch.float32, device="cuda")
+    gpu.ax(N, dev(torch, m.ggeo.astype(T)), dev(torch, m.D.astype(T).ravel()), dev(torch, q.astype(T)), Aq,
+           lambda0=dev(torch, np.array([1.3], dtype=T)), lambda1=dev(torch, np.array([2.0], dtype=T)),
+           poisson=False)
+    torch.cuda.synchronize()
+    assert rel(host(Aq), ref) < (1e-12 if T == np.float64 else 2e-5)
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 7, 9])
 def test_ax_golden_with_element_list(gpu, torch_mod, golden, N):
     torch = torch_mod
