@@ -35,7 +35,7 @@ struct AmgParams {
 
 // Host side of the hierarchy (kept for tests and the device upload).
 struct AmgHostLevel {
-  CsrHost A, P, R;               // P: n x nc, R = P^T
+  CsrHost A, P, R, RA;           // P: n x nc, R = P^T, R A (nc x n)
   std::vector<double> dinv;
   double omega = 0.0;            // 4 / (3 rho(D^-1 A))
   std::vector<double> inv;       // dense (pseudo-)inverse (last level only), row-major
@@ -44,11 +44,11 @@ std::vector<AmgHostLevel> amg_build(const CsrHost &A, const AmgParams &p);
 
 struct AmgDevLevel {
   int n = 0, nc = 0;
-  int laneA = 8, laneP = 8, laneR = 8;   // lanes per row of each matrix's SpMV
+  int laneA = 8, laneUp = 8, laneDown = 8;   // lanes per row of A, of P and A P, of R and R A
   bool dense = false;
-  double omega = 0.0;
-  DevBuf<int> arp, aci, prp, pci, rrp, rci;
-  DevBuf<double> av, pv, rv, dinv, inv;
+  DevBuf<int> arp, aci, prp, pci, rrp, rci, rarp, raci, aprp, apci;
+  DevBuf<double> av, pv, rv, rav, apv, inv;
+  DevBuf<double> w;                      // omega D^-1
   DevBuf<double> b, xa, xb, r;   // level vectors (coarser levels)
 };
 
@@ -63,10 +63,10 @@ struct Amg {
   int levels() const { return (int)lv.size(); }
 };
 
-// y = A x, and the fused forms used by the V-cycle and the coarse PCG
-enum { SPMV_Y = 0, SPMV_RES = 1, SPMV_ADD = 2, SPMV_JAC = 3 };
+// y = A x (SPMV_Y) or a damped-Jacobi sweep y = x + w .* (b - A x) (SPMV_JAC)
+enum { SPMV_Y = 0, SPMV_JAC = 1 };
 void csr_spmv(int mode, int n, const int *rp, const int *ci, const double *v, const double *x,
-              double *y, const double *b, const double *dinv, double omega, hipStream_t s, int lanes = 8);
+              double *y, const double *b, const double *w, hipStream_t s, int lanes = 8);
 // lanes per row suited to a matrix (8, or 64 for rows of 48+ entries on average)
 int csr_lanes(const CsrHost &A);
 
@@ -76,5 +76,16 @@ template <typename T>
 void rows_gather(int n, const int *first, const T *e, double *u, hipStream_t s);
 template <typename T>
 void rows_scatter(int64_t L, const int *rowOf, const double *u, T *e, hipStream_t s);
+
+// x = maxit AMG-preconditioned CG iterations for A x = r from x = 0, scattered to
+// the E-vector xout through rowOf (-1: 0); r, x, z, p, Ap, tmp: vectors of n
+// entries (r holds the right-hand side, all are overwritten), scratch: amg_pcg_scratch()
+// device doubles.  Enqueued on s only; an iteration whose residual is zero or NaN
+// changes nothing.
+size_t amg_pcg_scratch();
+template <typename T>
+void amg_pcg_fixed(Amg &amg, int n, const int *arp, const int *aci, const double *av, int maxit, double *r,
+                   double *x, double *z, double *p, double *Ap, double *tmp, double *scratch, int64_t L,
+                   const int *rowOf, T *xout, hipStream_t s);
 
 }  // namespace nrs

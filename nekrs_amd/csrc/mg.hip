@@ -389,7 +389,7 @@ struct CoarsePCG {
   int n = 0;
   Amg amg;
   DevBuf<int> rowOf, first, arp, aci;
-  DevBuf<double> av, ones, ru, xu, zu, pu, Apu, tmp;
+  DevBuf<double> av, ones, ru, xu, zu, pu, Apu, tmp, fixed;
   static constexpr int kChunkAmg = 2;
   ~CoarsePCG()
   {
@@ -407,7 +407,7 @@ struct CoarsePCG {
         pcg_precon_dots(*red, n, ones.get(), nullptr, ru.get(), zu.get(), Apu.get(), false, false, false,
                         scal.get(), s);
         pcg_update_p(n, zu.get(), pu.get(), scal.get(), s);
-        csr_spmv(SPMV_Y, n, arp.get(), aci.get(), av.get(), pu.get(), Apu.get(), nullptr, nullptr, 0.0, s);
+        csr_spmv(SPMV_Y, n, arp.get(), aci.get(), av.get(), pu.get(), Apu.get(), nullptr, nullptr, s);
         pcg_alpha(*red, n, ones.get(), pu.get(), Apu.get(), scal.get(), s);
         pcg_update_rx(*red, n, ones.get(), Apu.get(), pu.get(), ru.get(), xu.get(), 1.0, scal.get(), s);
       }
@@ -481,21 +481,9 @@ struct CoarsePCG {
       // BoomerAMG cycle count (coarseLevel.cpp:80-93)
       rows_gather<T>(n, first.get(), rhs, ru.get(), s);
       if (nullSpace) remove_mean(*red, n, nullptr, (double)n, ru.get(), scal.get(), S_TMP1, s);
-      fill<double>(n, 0.0, xu.get(), s);
-      fill<double>(n, 0.0, pu.get(), s);
-      wnorm(*red, n, ones.get(), ru.get(), 1.0, scal.get(), S_RDOTR, s);
-      pcg_init_device(scal.get(), 0.0, false, maxit, s);
-      for (int it = 0; it < maxit; ++it) {
-        amg.apply(ru.get(), zu.get(), tmp.get(), s);
-        pcg_precon_dots(*red, n, ones.get(), nullptr, ru.get(), zu.get(), Apu.get(), false, false, false,
-                        scal.get(), s);
-        pcg_update_p(n, zu.get(), pu.get(), scal.get(), s);
-        csr_spmv(SPMV_Y, n, arp.get(), aci.get(), av.get(), pu.get(), Apu.get(), nullptr, nullptr, 0.0, s);
-        pcg_alpha(*red, n, ones.get(), pu.get(), Apu.get(), scal.get(), s);
-        pcg_update_rx(*red, n, ones.get(), Apu.get(), pu.get(), ru.get(), xu.get(), 1.0, scal.get(), s);
-      }
+      amg_pcg_fixed<T>(amg, n, arp.get(), aci.get(), av.get(), maxit, ru.get(), xu.get(), zu.get(), pu.get(),
+                       Apu.get(), tmp.get(), fixed.get(), L, rowOf.get(), xout, s);
       lastIters = maxit;
-      rows_scatter<T>(L, rowOf.get(), xu.get(), xout, s);
       return;
     }
     rows_gather<T>(n, first.get(), rhs, ru.get(), s);
@@ -604,6 +592,7 @@ struct CoarsePCG {
     amg.setup(A, ap);
     amgMode = true;
     deviceOnly = !(tol > 0.0);
+    if (deviceOnly) fixed.alloc(amg_pcg_scratch());
     NRS_CHECK(!deviceOnly || (maxit >= 1 && maxit <= 64),
               "coarse AMG with coarseTol <= 0 runs exactly coarseMaxIter (1..64) iterations");
   }
