@@ -728,8 +728,19 @@ int elliptic_krylov(nrs_elliptic *el, double *r, double *x, double res0, double 
   // flag says the iteration has stopped (converged or maxIter), so x, r and
   // the count are those of checking after each iteration.
   const int perCheck = (none || o.preconditioner == NRS_PRECON_JACOBI) ? 4 : 1;
+  // plain PCG with the preconditioner inside the vector kernels: the first
+  // iteration's dots here, the later ones' with the residual update
+  const bool direct = (none || jacobi) && !flexible;
+  const double *invDiag = none ? nullptr : el->invDiagA.get();
+  if (direct) pcg_precon_dots(R, L, w, invDiag, r, z, Ap, jacobi, false, none, scal, s);
   for (;;) {
     for (int b = 0; b < perCheck; ++b) {
+      if (direct) {
+        pcg_update_p_direct(L, invDiag, r, p, scal, s);
+        elliptic_operator(el, p, Ap, true, s);
+        pcg_step(R, L, w, invDiag, Ap, p, r, x, resNormFactor, scal, s);
+        continue;
+      }
       if (!none && !jacobi) {   // timed only with perCheck = 1: the events are read after the readback
         if (timed && perCheck == 1) NRS_HIP(hipEventRecord(el->evPre0, s));
         elliptic_preconditioner(el, r, z, s);

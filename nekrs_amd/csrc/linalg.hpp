@@ -22,7 +22,7 @@ enum Scalar : int {
 struct Reducer {
   static constexpr int kBlocks = 1024;   // upper bound on the partials grid
   static constexpr int kThreads = 256;
-  DevBuf<double> partials;               // [kBlocks * 2]
+  DevBuf<double> partials;               // [kBlocks * 3]
   Reducer();
 };
 
@@ -66,6 +66,14 @@ void pcg_alpha(Reducer &R, int64_t n, const double *w, const double *p, const do
 // r -= alpha Ap; x += alpha p; rdotr = sqrt(<r,r>_w * resNormFactor)
 void pcg_update_rx(Reducer &R, int64_t n, const double *w, const double *Ap, const double *p,
                    double *r, double *x, double resNormFactor, double *scal, hipStream_t s);
+// The iteration of plain PCG without a preconditioner (invDiag null) or with
+// Jacobi, after pcg_precon_dots has set up the first one: p = z + beta p with
+// z = invDiag .* r formed on the way; then, once Ap is known, alpha, the updates
+// of x and r, the norm and the next iteration's beta in three launches.
+void pcg_update_p_direct(int64_t n, const double *invDiag, const double *r, double *p, const double *scal,
+                         hipStream_t s);
+void pcg_step(Reducer &R, int64_t n, const double *w, const double *invDiag, const double *Ap, const double *p,
+              double *r, double *x, double resNormFactor, double *scal, hipStream_t s);
 // linAlg_t reductions over n entries of nf fields spaced off apart (op: nrs_reduction);
 // partials: device scratch of at least reduce_partials_needed(n) doubles; out: one
 // device double.  Deterministic: fixed per-thread order, fixed tree order.

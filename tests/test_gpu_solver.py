@@ -80,6 +80,23 @@ def test_solve_small_vs_oracle(gpu, torch_mod, orc, solver, precon):
         assert rel(host(x), xo) <= 1e-8
 
 
+@pytest.mark.parametrize("precon", ["jacobi", "none"])
+@pytest.mark.parametrize("shape,N", [((2, 1, 1), 2), ((3, 2, 2), 4), ((7, 6, 5), 6)])
+def test_pcg_iterates_vs_oracle(gpu, torch_mod, orc, precon, shape, N):
+    """The first PCG iterates, where rounding has not been amplified yet: vectors
+    shorter than a block, with a ragged end, and of more entries than threads.
+    1e-12 = 1e4 roundings of sums of up to 72030 entries over 4 iterations."""
+    torch = torch_mod
+    for its in (1, 4):
+        eg, eo = both(gpu, orc, *shape, N, "kershaw", precon=precon, tol=1e-30, max_iter=its)
+        rhs = np.random.default_rng(N).uniform(-1, 1, eg.Nlocal)
+        xo, _ = eo.solve(rhs, precon=precon, tol=1e-30, maxit=its)
+        x = torch.zeros(eg.Nlocal, dtype=torch.float64, device="cuda")
+        st = eg.solve(dev(torch, rhs), x)
+        print(precon, shape, N, its, "rel", rel(host(x), xo))
+        assert st["iterations"] == its and rel(host(x), xo) <= 1e-12
+
+
 def test_solve_nonzero_initial_guess(gpu, torch_mod, orc):
     torch = torch_mod
     eg, eo = both(gpu, orc, 3, 2, 2, 4, "kershaw", tol=1e-10, max_iter=500)
