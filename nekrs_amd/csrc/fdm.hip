@@ -1004,6 +1004,9 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
 // elements: 47.3 -> 33 us a launch (counters: matrix cores busy 45 % of it, VALU
 // 25 %, the rest the loads at the start of each wave; a persistent wave that
 // loads the next element ahead, 1 to 5 blocks per CU, was 5-60 % slower).
+// SUB: the boxes of u - sub, the difference kept in diff where that is not null;
+// results times scale.  A Chebyshev step's residual update and first scaling then
+// need no passes of their own (9.5 us each there, 1.5 us here).
 template <int NQ> struct FdmF32Cfg {
   static constexpr int NL = NQ + 2;
   static constexpr int NT = (NL * NL + 15) / 16;     // tiles of 16 rows
@@ -1019,11 +1022,11 @@ template <int NQ> struct FdmF32Cfg {
   static_assert(NL <= 12 && PS % 4 == 0, "one 16-wide tile of outputs, aligned rows");
 };
 
-template <int NQ, bool ASM>
+template <int NQ, bool ASM, bool SUB>
 __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kernel(
     int E, const float *__restrict__ u, const float *__restrict__ S, const double *__restrict__ lam,
     double2 helm, const int4 *__restrict__ gmap, float *__restrict__ out, float *__restrict__ gout,
-    const uint32_t *__restrict__ mbits)
+    const uint32_t *__restrict__ mbits, const float *__restrict__ sub, float *__restrict__ diff, float scale)
 {
   using C = FdmF32Cfg<NQ>;
   constexpr int NL = C::NL, NT = C::NT, KS = C::KS, PS = C::PS, NP = NQ * NQ * NQ, NQ2 = NQ * NQ;
@@ -1057,13 +1060,24 @@ __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kern
     const unsigned n = lane + 64 * t;
     vi[t] = (n < NP) ? ue[n] : 0.f;
   }
+  float vs[SUB ? RI : 1], ns[SUB ? 6 : 1][RG];       // the same nodes of sub
+  if constexpr (SUB) {
+#pragma unroll
+    for (int t = 0; t < RI; ++t) {
+      const unsigned n = lane + 64 * t;
+      vs[t] = (n < NP) ? sub[(int64_t)e * NP + n] : 0.f;
+    }
+  }
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
     const int4 gm = gmap[(int64_t)e * 6 + f];
 #pragma unroll
     for (int t = 0; t < RG; ++t) {
       const int n = lane + 64 * t;
-      nb[f][t] = (gm.x >= 0 && n < NQ2) ? u[(unsigned)(gm.x + (n % NQ) * gm.y + (n / NQ) * gm.z)] : 0.f;
+      const bool on = gm.x >= 0 && n < NQ2;
+      const unsigned q = (unsigned)(gm.x + (n % NQ) * gm.y + (n / NQ) * gm.z);
+      nb[f][t] = on ? u[q] : 0.f;
+      if constexpr (SUB) ns[f][t] = on ? sub[q] : 0.f;
     }
   }
   const float *Se = S + (int64_t)e * 3 * NL * NL;
@@ -1092,6 +1106,21 @@ __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kern
   for (int t = 0; t < RL; ++t)
     if (lane + 64 * t < 16 * NT) lyz[lane + 64 * t] = ly[t] + lz[t];
   wave_lds_sync();
+  if constexpr (SUB) {
+#pragma unroll
+    for (int t = 0; t < RI; ++t) vi[t] -= vs[t];
+#pragma unroll
+    for (int f = 0; f < 6; ++f)
+#pragma unroll
+      for (int t = 0; t < RG; ++t) nb[f][t] -= ns[f][t];
+    if (diff) {
+#pragma unroll
+      for (int t = 0; t < RI; ++t) {
+        const unsigned n = lane + 64 * t;
+        if (n < NP) diff[(int64_t)e * NP + n] = vi[t];
+      }
+    }
+  }
 #pragma unroll
   for (int t = 0; t < RI; ++t) {
     const int n = lane + 64 * t;
@@ -1173,7 +1202,7 @@ __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kern
   for (int t = 0; t < RI; ++t) {
     const unsigned n = lane + 64 * t;
     if (n < NP) {
-      float v = X[at(n / NQ2 + 1, (n / NQ) % NQ + 1, n % NQ + 1)];
+      float v = X[at(n / NQ2 + 1, (n / NQ) % NQ + 1, n % NQ + 1)] * scale;
       if (mb) {   // the two mask words of these 64 nodes, by scalar loads
         const uint32_t w0 = mb[2 * t], w1 = mb[2 * t + 1 < NW ? 2 * t + 1 : 2 * t];
         if (((lane < 32 ? w0 : w1) >> (lane & 31)) & 1u) v = 0.f;
@@ -1188,7 +1217,7 @@ __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kern
 #pragma unroll
       for (int t = 0; t < RG; ++t) {
         const int n = lane + 64 * t;
-        if (n < NQ2) ge[f * NQ2 + n] = X[face_at(f, n % NQ, n / NQ, 0)];
+        if (n < NQ2) ge[f * NQ2 + n] = X[face_at(f, n % NQ, n / NQ, 0)] * scale;
       }
   }
 }
@@ -1211,15 +1240,16 @@ void launch_fdm_mfma_nq(bool ras, int E, const float *u, const uint16_t *S16, co
 
 template <typename T, int NQ>
 void launch_fdm_nq(bool ras, int E, const T *u, const T *S, const double *lam, double2 helm, const int4 *gmap,
-                   T *out, T *gout, const uint32_t *mbits, hipStream_t s)
+                   T *out, T *gout, const uint32_t *mbits, const T *sub, T *diff, T scale, hipStream_t s)
 {
   if constexpr (std::is_same<T, float>::value) {
     constexpr int W = FdmF32Cfg<NQ>::WAVES;
     const unsigned grid = (unsigned)((E + W - 1) / W);
-    if (ras)
-      fdm_f32_kernel<NQ, false><<<grid, 64 * W, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
-    else
-      fdm_f32_kernel<NQ, true><<<grid, 64 * W, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits);
+#define FDM(A_, S_)                                                                                     \
+  fdm_f32_kernel<NQ, A_, S_><<<grid, 64 * W, 0, s>>>(E, u, S, lam, helm, gmap, out, gout, mbits, sub, diff, scale)
+    if (ras) { if (sub) FDM(false, true); else FDM(false, false); }
+    else { if (sub) FDM(true, true); else FDM(true, false); }
+#undef FDM
   } else {
     using C = FdmCfg<NQ>;
     const unsigned grid = (unsigned)((E + C::EPB - 1) / C::EPB);
@@ -1379,9 +1409,11 @@ static void fdm_mfma_boxes(int Nq, int fmt, bool ras, int E, const float *u, con
 }
 
 template <typename T>
-void Schwarz<T>::apply(const T *u, T *Su, hipStream_t s)
+void Schwarz<T>::apply(const T *u, T *Su, hipStream_t s, const T *sub, T *diff, T scale)
 {
-  NRS_CHECK((const void *)u != (const void *)Su, "schwarz: input and output must differ");
+  NRS_CHECK((const void *)u != (const void *)Su && sub != Su, "schwarz: input and output must differ");
+  NRS_CHECK(takes_sub() || (!sub && scale == T(1)), "schwarz: no difference or scale on this path");
+  NRS_CHECK(!diff || (sub && diff != u && diff != sub && diff != Su), "schwarz: the difference needs a vector of its own");
   T *out = ras ? Su : boxOut.get();
   T *gout = ras ? nullptr : ghostOut.get();
   if constexpr (std::is_same<T, float>::value) {
@@ -1406,7 +1438,7 @@ void Schwarz<T>::apply(const T *u, T *Su, hipStream_t s)
 #define NRS_FDM_CASE(NQ_)                                                                      \
   case NQ_:                                                                                    \
     launch_fdm_nq<T, NQ_>(ras, E, u, S.get(), lam.get(), make_double2(helm0, helm1), gmap.get(), out, gout,       \
-                          maskBits, s);                                                                        \
+                          maskBits, sub, diff, scale, s);                                                      \
     if (!ras) launch_post_nq<T, NQ_>(E, boxOut.get(), ghostOut.get(), smap.get(), wts.get(), Su, maskBits, s);   \
     break;
   switch (Nq) {

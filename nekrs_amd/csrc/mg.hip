@@ -204,19 +204,19 @@ __global__ void jacobi_first_kernel(int64_t n, T invTheta, const T *__restrict__
   }
 }
 
-// updateFourthKindChebyshev (kernels/elliptic/updateFourthKindChebyshev.okl:5-25)
-// split in two: its residual update r -= A d runs before the smoother (which
-// reads r), and its x += beta d is deferred into the direction update after
-// the smoother, which reads d anyway.  X0: r = rin - A d with rin the
-// right-hand side (a zero start, where r is not yet formed).
-template <typename T, bool X0>
-__global__ void cheby4_res_kernel(int64_t n, const T *__restrict__ Ad, const T *__restrict__ rin,
-                                  T *__restrict__ r)
+// d = a - b (d may be a or b)
+template <typename T>
+__global__ void diff_kernel(int64_t n, const T *a, const T *b, T *d)
 {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    r[i] = (X0 ? rin[i] : r[i]) - Ad[i];
+    d[i] = a[i] - b[i];
 }
 
+// updateFourthKindChebyshev (kernels/elliptic/updateFourthKindChebyshev.okl:5-25)
+// split in two: its residual update r -= A d goes with the smoother that reads
+// r, and its x += beta d is deferred into the direction update after the
+// smoother, which reads d anyway.
+//
 // After the smoother: x = x + beta d (the deferred half of the update; X0: x
 // taken as zero, not read), then d = rC SAd + dC d -- or, on the last step
 // (LAST), x = beta_last (rC SAd + dC d) + x with d not stored: the roundings
@@ -603,6 +603,7 @@ struct MGImpl final : MGSolver {
   nrs_elliptic *el = nullptr;
   std::vector<std::unique_ptr<Level<T>>> levels;
   DevBuf<T> sRes, sAd, sD, sTmp;  // shared smoother work vectors (finest size)
+  DevBuf<T> sOut;                 // one more where the Schwarz kernel forms the residual
   DevBuf<T> rP, zP;               // level-0 FP32 copies of r and z
   DevBuf<T> cornersT;             // element corners [E][3][8] of a trilinear mesh (else empty)
   std::unique_ptr<CoarsePCG> coarse;
@@ -644,6 +645,25 @@ struct MGImpl final : MGSolver {
     else k_wmul<T>(l.L, l.invDiagA.get(), in, out, s);
   }
 
+  // Su = scale * S(a - b), or scale * S(a) with b null.  Schwarz boxes that take a
+  // difference form it as they load (diff: kept there, null: not kept); otherwise
+  // it is written to tmp first (which may be a or b).  Returns where the
+  // difference is.
+  T *smoother_sub(Level<T> &l, const T *a, const T *b, T *diff, T *tmp, T *Su, T scale, hipStream_t s)
+  {
+    if (l.schwarz && l.schwarz->takes_sub()) {
+      l.schwarz->apply(a, Su, s, b, diff, scale);
+      return diff;
+    }
+    if (b) {
+      diff_kernel<T><<<kgrid(l.L), KB, 0, s>>>(l.L, a, b, tmp);
+      NRS_LAUNCH_CHECK();
+    }
+    smootherS(l, b ? tmp : a, Su, s);
+    if (scale != T(1)) k_axpby<T>(l.L, scale, Su, T(0), Su, s);
+    return tmp;
+  }
+
   // smoothChebyshev (ellipticMultiGridLevel.cpp:144-210).  The reference
   // smooths res and Ad in place; here S writes to a spare vector whose role is
   // swapped with the input's.  Scalars are formed in FP64 and rounded to T.
@@ -670,13 +690,8 @@ struct MGImpl final : MGSolver {
     const bool jac = !l.schwarz;
     // x = 0 with at least one update step: that step takes x as zero (no fill)
     const bool x0 = xIsZero && deg > 1;
-    if (xIsZero) {
-      if (!x0) fill<T>(l.L, T(0), x, s);
-      if (!jac) k_axpby<T>(l.L, T(1), rhs, T(0), res, s);   // res = rhs
-    } else {
-      op(l, x, res, s);
-      if (!jac) k_axpby<T>(l.L, T(1), rhs, T(-1), res, s);
-    }
+    if (!xIsZero) op(l, x, res, s);
+    else if (!x0) fill<T>(l.L, T(0), x, s);
     if (jac) {
       if (xIsZero)
         jacobi_first_kernel<T, false><<<kgrid(l.L), KB, 0, s>>>(l.L, invTheta, l.invDiagA.get(), rhs,
@@ -687,7 +702,7 @@ struct MGImpl final : MGSolver {
       NRS_LAUNCH_CHECK();
       std::swap(res, spare);
     } else {
-      smootherS(l, res, spare, s);
+      smoother_sub(l, rhs, xIsZero ? nullptr : res, nullptr, res, spare, T(1), s);
       std::swap(res, spare);
       k_axpby<T>(l.L, invTheta, res, T(0), d, s);
     }
@@ -730,38 +745,35 @@ struct MGImpl final : MGSolver {
     const double rho = l.lmax;
     const uint32_t *lm = last_mask(l);
     T *res = sRes.get(), *Ad = sAd.get(), *d = sD.get();
+    // the smoother's result, and the next residual where it is formed in the boxes
+    T *Su = sOut.get() ? sOut.get() : Ad, *next = sTmp.get();
     // x = 0 with at least one update step: the first step treats x as zero and
     // takes the residual from rhs, so neither is written beforehand
     const bool x0 = xIsZero && deg > 1;
-    if (xIsZero) {
-      if (!x0) {
-        fill<T>(l.L, T(0), x, s);
-        k_axpby<T>(l.L, T(1), rhs, T(0), res, s);   // res = rhs
-      }
-    } else {
-      op(l, x, res, s);
-      k_axpby<T>(l.L, T(1), rhs, T(-1), res, s);
-    }
-    smootherS(l, x0 ? rhs : res, Ad, s);
     const T coeff = T(4.0 / (3.0 * rho));
-    k_axpby<T>(l.L, coeff, Ad, T(0), d, s);
+    const T *r = rhs;                       // the residual
+    if (xIsZero) {
+      if (!x0) fill<T>(l.L, T(0), x, s);
+      smoother_sub(l, rhs, nullptr, nullptr, nullptr, d, coeff, s);
+    } else {
+      op(l, x, Ad, s);
+      r = smoother_sub(l, rhs, Ad, deg > 1 ? res : nullptr, res, d, coeff, s);
+    }
     for (int k = 1; k < deg; ++k) {
       op(l, d, Ad, s);
       const bool first0 = k == 1 && x0, last = k + 1 == deg;
       const unsigned g = kgrid(l.L);
-      if (first0) cheby4_res_kernel<T, true><<<g, KB, 0, s>>>(l.L, Ad, rhs, res);
-      else cheby4_res_kernel<T, false><<<g, KB, 0, s>>>(l.L, Ad, res, res);
-      NRS_LAUNCH_CHECK();
-      smootherS(l, res, Ad, s);
+      r = smoother_sub(l, r, Ad, last ? nullptr : next, res, Su, T(1), s);
+      if (r == next) std::swap(res, next);
       const T dC = T((2.0 * k - 1.0) / (2.0 * k + 3.0));
       const T rC = T((8.0 * k + 4.0) / ((2.0 * k + 3.0) * rho));
       const T b = betas[k - 1], bl = betas.back();
       // x += beta_(k-1) d deferred to here, with the direction update (and, on
       // the last step, the final x += beta_last d)
-      if (first0 && last) cheby4_dir_kernel<T, true, true><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Ad, d, x, lm, l.Np);
-      else if (first0) cheby4_dir_kernel<T, true, false><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Ad, d, x);
-      else if (last) cheby4_dir_kernel<T, false, true><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Ad, d, x, lm, l.Np);
-      else cheby4_dir_kernel<T, false, false><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Ad, d, x);
+      if (first0 && last) cheby4_dir_kernel<T, true, true><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Su, d, x, lm, l.Np);
+      else if (first0) cheby4_dir_kernel<T, true, false><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Su, d, x);
+      else if (last) cheby4_dir_kernel<T, false, true><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Su, d, x, lm, l.Np);
+      else cheby4_dir_kernel<T, false, false><<<g, KB, 0, s>>>(l.L, b, rC, dC, bl, Su, d, x);
       NRS_LAUNCH_CHECK();
     }
     if (deg == 1) k_axpby<T>(l.L, betas.back(), d, T(1), x, s);
@@ -1207,6 +1219,7 @@ struct MGImpl final : MGSolver {
     }
     const int64_t L0 = levels[0]->L;
     sRes.alloc(L0); sAd.alloc(L0); sD.alloc(L0); sTmp.alloc(L0);
+    if (cheby == CHEBY_OPT4 && levels[0]->schwarz && levels[0]->schwarz->takes_sub()) sOut.alloc(L0);
     cycleGraphs = o.useGraphs != 0;
     if (cycleGraphs && std::is_same<T, double>::value) { rIn.alloc(L0); zOut.alloc(L0); }
     if (!std::is_same<T, double>::value) { rP.alloc(L0); zP.alloc(L0); }

@@ -130,6 +130,27 @@ def test_mg_schwarz_fcg_vs_oracle(gpu, torch_mod, orc, cheby, S, degree):
 
 
 @pytest.mark.parametrize("S", ["asm", "ras"])
+@pytest.mark.parametrize("prec,cheby,degree", [(0, "opt4", 1), (0, "opt4", 2), (0, "opt4", 5), (0, "cheby1", 1),
+                                               (0, "cheby1", 3), (1, "opt4", 1), (1, "opt4", 4), (1, "cheby1", 2)])
+def test_chebyshev_degrees_vs_oracle(gpu, torch_mod, orc, prec, cheby, degree, S):
+    """One V-cycle with the residual formed inside the boxes (FP32) and beside
+    them (FP64) at every length of the Chebyshev loop: the bars of a V-cycle,
+    2e-4 in FP32 and 1e-9 in FP64.  One smoothed level: its Chebyshev interval is
+    the oracle's to 1e-13 (an order-2 level's differs by 4e-4, which alone moves a
+    cycle by 2e-5)."""
+    torch = torch_mod
+    eg, eo, om = pair(gpu, orc, (4, 3, 3), 4, [4, 1], cheby, S, prec=prec, degree=degree)
+    r = np.random.default_rng(degree).uniform(-1, 1, eg.Nlocal)
+    r[eo.maskIds] = 0
+    r = eo.ogs.gs(r, "add")
+    z = torch.zeros(eg.Nlocal, dtype=torch.float64, device="cuda")
+    eg.preconditioner(dev(torch, r), z)
+    e = rel(z.cpu().numpy(), om.apply(r))
+    print(prec, cheby, degree, S, "rel", e)
+    assert e < (2e-4 if prec == 0 else 1e-9)
+
+
+@pytest.mark.parametrize("S", ["asm", "ras"])
 def test_pure_schwarz_fcg_vs_oracle(gpu, torch_mod, orc, S):
     """ASM / RAS without Chebyshev (no post-smoothing) on a sine-deformed box."""
     import oracle.mg as omg
