@@ -312,3 +312,31 @@ def test_mask_kernel(gpu, torch_mod):
     out = host(v)
     assert np.all(out[[0, 5, 999, 500]] == 0)
     assert np.count_nonzero(out == 0) == 4
+
+
+@pytest.mark.parametrize("Nf,Nc", [(2, 1), (3, 1), (3, 2), (4, 1), (4, 3), (5, 1), (5, 2), (5, 4), (6, 1), (6, 5)])
+@pytest.mark.parametrize("E", [1, 6])
+def test_transfer_order_pairs(gpu, torch_mod, Nf, Nc, E):
+    """Both transfers for the orders one wave takes and the first above them, with
+    a block that is not full.  Three sums of at most 7 terms: 32 roundings of
+    the sum of absolute values."""
+    torch = torch_mod
+    rng = np.random.default_rng(10 * Nf + Nc)
+    nf, nc = Nf + 1, Nc + 1
+    R, qf, qc = rng.uniform(-1, 1, (nc, nf)), rng.uniform(-1, 1, (E, nf, nf, nf)), rng.uniform(-1, 1, (E, nc, nc, nc))
+
+    def down(A, q):
+        return np.einsum("ck,bj,ai,ekji->ecba", A, A, A, q)
+
+    for dt, npd in ((torch.float64, np.float64), (torch.float32, np.float32)):
+        eps = np.finfo(npd).eps
+        Rd, f, c = (torch.from_numpy(a.astype(npd).ravel()).cuda() for a in (R, qf, qc))
+        R64, f64, c64 = (a.astype(npd).astype(np.float64) for a in (R, qf, qc))
+        out = torch.zeros(E * nc ** 3, dtype=dt, device="cuda")
+        gpu.coarsen(Nf, Nc, Rd, f, out)
+        err = np.abs(out.cpu().numpy() - down(R64, f64).ravel())
+        assert np.all(err <= 32 * eps * down(np.abs(R64), np.abs(f64)).ravel())
+        acc = f.clone()
+        gpu.prolongate(Nf, Nc, Rd, c, acc)
+        up, bound = f64 + down(R64.T, c64), np.abs(f64) + down(np.abs(R64.T), np.abs(c64))
+        assert np.all(np.abs(acc.cpu().numpy() - up.ravel()) <= 32 * eps * bound.ravel())
