@@ -334,6 +334,13 @@ def test_pgmres_vs_oracle(gpu, torch_mod, orc, solver, precon, restart):
     assert rel(host(x), xo) <= 1e-8
 
 
+@pytest.mark.parametrize("restart", [4, 16, 17, 32])
+def test_pgmres_vector_counts(gpu, torch_mod, orc, restart):
+    """The inner products' groups of four vectors full, with a remainder, and at
+    the most vectors there are (every count up to the restart length is passed)."""
+    test_pgmres_vs_oracle(gpu, torch_mod, orc, "gmres", "jacobi", restart)
+
+
 def test_pgmres_block_three_fields(gpu, torch_mod, orc):
     import oracle.mg as omg
     torch = torch_mod
