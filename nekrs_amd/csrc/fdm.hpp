@@ -53,8 +53,8 @@ struct Schwarz {
   int64_t Nmasked = 0;
   const int *maskIds = nullptr;
   // [E][ceil(Np/32)] Dirichlet mask bits of the level's nodes: the ASM
-  // overlap kernel and the SIMT box solve store the masked nodes of Su as zero
-  // (null, or RAS on the matrix cores: the mask runs as its own pass over
+  // overlap kernel and the FP32 and FP64 box solves store the masked nodes of Su as zero
+  // (null, or RAS with 16-bit operators: the mask runs as its own pass over
   // maskIds).  The masked nodes must be in no row of ogs, as the level's
   // handles are built.
   const uint32_t *maskBits = nullptr;
