@@ -695,11 +695,17 @@ template <int NQ> struct MfmaCfg {
 // of the current one, and the results of an element are staged in LDS and
 // written out (as whole rows) only after the next element's loads have
 // arrived, so no wait on outstanding stores sits in front of the prefetch.
-template <int NQ, int FMT, bool ASM>
+// SUB: the boxes of u - sub, the difference kept in diff unless null; results
+// times scale (as the FP32 form below).  30 more registers (order 7, RAS: 127 ->
+// 157, a wave per SIMD less) against a pass over three vectors for each step: V-cycles
+// 20^3 order 7 RAS 830 us -> 782, 17x19x18 order 5 ASM 655 -> 628, 32^3 order 7
+// 2608 -> 2550; FP16 12^3 order 7 ASM 496 -> 458.
+template <int NQ, int FMT, bool ASM, bool SUB>
 __global__ __launch_bounds__(256) void fdm_mfma_kernel(
     int E, const float *__restrict__ u, const uint16_t *__restrict__ S16,
     const float *__restrict__ lam, float2 helm, const int4 *__restrict__ gmap,
-    float *__restrict__ out, float *__restrict__ gout)
+    float *__restrict__ out, float *__restrict__ gout, const float *__restrict__ sub, float *__restrict__ diff,
+    float scale)
 {
   using C = MfmaCfg<NQ>;
   constexpr int NL = C::NL, PS = C::PS, RW = C::RW, BUF = C::BUF, NP = NQ * NQ * NQ, NQ2 = NQ * NQ;
@@ -726,6 +732,8 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
 
   // ---- prefetch state of the next element
   float pvi[RI][NQ], pown[6][RG], pnb[6][RG], plx[4], plz, ply[NL];
+  constexpr int RB = SUB ? RI : 1, GB = SUB ? 6 : 1;
+  float svi[RB][NQ], sown[GB][RG], snb[GB][RG];   // SUB: the same nodes of sub
   uint4 ps[RS];
   int4 pgm[6];
   auto load_a = [&](int en) {
@@ -735,13 +743,19 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
       const int n = lane + 64 * t;
 #pragma unroll
       for (int i = 0; i < NQ; ++i) pvi[t][i] = (n < NQ2) ? ue[n * NQ + i] : 0.f;
+      if constexpr (SUB) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) svi[t][i] = (n < NQ2) ? sub[(int64_t)en * NP + n * NQ + i] : 0.f;
+      }
     }
 #pragma unroll
     for (int f = 0; f < 6; ++f)
 #pragma unroll
       for (int t = 0; t < RG; ++t) {
         const int n = lane + 64 * t;
-        pown[f][t] = (n < NQ2) ? ue[face_node(f, n % NQ, n / NQ, 1, NQ - 1)] : 0.f;
+        const int q = face_node(f, n % NQ, n / NQ, 1, NQ - 1);
+        pown[f][t] = (n < NQ2) ? ue[q] : 0.f;
+        if constexpr (SUB) sown[f][t] = (n < NQ2) ? sub[(int64_t)en * NP + q] : 0.f;
       }
     const uint4 *Se = reinterpret_cast<const uint4 *>(S16 + (int64_t)en * SST);
 #pragma unroll
@@ -765,7 +779,10 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
 #pragma unroll
       for (int t = 0; t < RG; ++t) {
         const int n = lane + 64 * t;
-        pnb[f][t] = (gm.x >= 0 && n < NQ2) ? u[gm.x + (n % NQ) * gm.y + (n / NQ) * gm.z] : 0.f;
+        const bool on = gm.x >= 0 && n < NQ2;
+        const int q = gm.x + (n % NQ) * gm.y + (n / NQ) * gm.z;
+        pnb[f][t] = on ? u[q] : 0.f;
+        if constexpr (SUB) snb[f][t] = on ? sub[q] : 0.f;
       }
     }
   };
@@ -788,11 +805,30 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
 #pragma unroll
     for (int t = 0; t < RI; ++t)
 #pragma unroll
-      for (int i = 0; i < NQ; ++i) vi[t][i] = pvi[t][i];
+      for (int i = 0; i < NQ; ++i) {
+        if constexpr (SUB) vi[t][i] = pvi[t][i] - svi[t][i];
+        else vi[t][i] = pvi[t][i];
+      }
 #pragma unroll
     for (int f = 0; f < 6; ++f)
 #pragma unroll
-      for (int t = 0; t < RG; ++t) vg[f][t] = (pown[f][t] + pnb[f][t]) - pown[f][t];   // fusedFDM.c:47-104
+      for (int t = 0; t < RG; ++t) {
+        float own = pown[f][t], nb = pnb[f][t];
+        if constexpr (SUB) { own -= sown[f][t]; nb -= snb[f][t]; }
+        vg[f][t] = (own + nb) - own;   // fusedFDM.c:47-104
+      }
+    if constexpr (SUB) {
+      if (diff) {
+#pragma unroll
+        for (int t = 0; t < RI; ++t) {
+          const int n = lane + 64 * t;
+          if (n < NQ2) {
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) diff[(int64_t)e * NP + n * NQ + i] = vi[t][i];
+          }
+        }
+      }
+    }
 #pragma unroll
     for (int t = 0; t < RS; ++t) sr[t] = ps[t];
 #pragma unroll
@@ -940,7 +976,7 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
     contract(X, bb[1]); rescale(); store(Y);          // T5[j][i][p]
     contract(Y, bb[2]);                               // out[k][j][i]: k = c, j = a, i = 4g+q
     wave_lds_sync();                                  // T5 fully read: Y becomes the staging area
-    const float inv = 1.f / sc;
+    const float inv = SCALE ? scale / sc : scale;     // sc = 1 without block scaling
     if (c < NQ) {
 #pragma unroll
       for (int a = 0; a < NQ; ++a)
@@ -1226,15 +1262,17 @@ __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kern
 // the prefetch has something to overlap)
 template <int NQ, int FMT>
 void launch_fdm_mfma_nq(bool ras, int E, const float *u, const uint16_t *S16, const float *lam,
-                        float2 helm, const int4 *gmap, float *out, float *gout, int epw, hipStream_t s)
+                        float2 helm, const int4 *gmap, float *out, float *gout, const float *sub, float *diff,
+                        float scale, int epw, hipStream_t s)
 {
   using C = MfmaCfg<NQ>;
   const int64_t perBlock = (int64_t)C::WAVES * std::max(1, epw);
   const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((E + perBlock - 1) / perBlock, 65536));
-  if (ras)
-    fdm_mfma_kernel<NQ, FMT, false><<<grid, 64 * C::WAVES, 0, s>>>(E, u, S16, lam, helm, gmap, out, gout);
-  else
-    fdm_mfma_kernel<NQ, FMT, true><<<grid, 64 * C::WAVES, 0, s>>>(E, u, S16, lam, helm, gmap, out, gout);
+#define FDM(A_, S_)                                                                                     \
+  fdm_mfma_kernel<NQ, FMT, A_, S_><<<grid, 64 * C::WAVES, 0, s>>>(E, u, S16, lam, helm, gmap, out, gout, sub, diff, scale)
+  if (ras) { if (sub) FDM(false, true); else FDM(false, false); }
+  else { if (sub) FDM(true, true); else FDM(true, false); }
+#undef FDM
   NRS_LAUNCH_CHECK();
 }
 
@@ -1389,15 +1427,15 @@ void Schwarz<T>::setup(int N_, int E_, bool ras_, int prec, const std::vector<do
 
 // the matrix-core box solves of one Schwarz level (FP32 vectors)
 static void fdm_mfma_boxes(int Nq, int fmt, bool ras, int E, const float *u, const uint16_t *S16,
-                           const float *lam, float2 helm, const int4 *gmap, float *out, float *gout, int epw,
-                           hipStream_t s)
+                           const float *lam, float2 helm, const int4 *gmap, float *out, float *gout,
+                           const float *sub, float *diff, float scale, int epw, hipStream_t s)
 {
 #define NRS_FDM_MFMA_CASE(NQ_)                                                                 \
   case NQ_:                                                                                    \
     if (fmt == NRS_FDM_BF16)                                                                   \
-      launch_fdm_mfma_nq<NQ_, NRS_FDM_BF16>(ras, E, u, S16, lam, helm, gmap, out, gout, epw, s);     \
+      launch_fdm_mfma_nq<NQ_, NRS_FDM_BF16>(ras, E, u, S16, lam, helm, gmap, out, gout, sub, diff, scale, epw, s);     \
     else                                                                                       \
-      launch_fdm_mfma_nq<NQ_, NRS_FDM_F16>(ras, E, u, S16, lam, helm, gmap, out, gout, epw, s);      \
+      launch_fdm_mfma_nq<NQ_, NRS_FDM_F16>(ras, E, u, S16, lam, helm, gmap, out, gout, sub, diff, scale, epw, s);      \
     break;
   switch (Nq) {
     NRS_FDM_MFMA_CASE(2) NRS_FDM_MFMA_CASE(3) NRS_FDM_MFMA_CASE(4) NRS_FDM_MFMA_CASE(5)
@@ -1419,7 +1457,8 @@ void Schwarz<T>::apply(const T *u, T *Su, hipStream_t s, const T *sub, T *diff, 
   if constexpr (std::is_same<T, float>::value) {
     if (fdmPrecision != NRS_FDM_F32) {
       const int epw = tuned(TUNE_FDM, N, fdmPrecision, E, 4);
-      fdm_mfma_boxes(Nq, fdmPrecision, ras, E, u, S16.get(), lam32.get(), helm32(), gmap.get(), out, gout, epw, s);
+      fdm_mfma_boxes(Nq, fdmPrecision, ras, E, u, S16.get(), lam32.get(), helm32(), gmap.get(), out, gout, sub, diff,
+                     scale, epw, s);
       if (!ras) {
 #define NRS_FDM_POST_CASE(NQ_)                                                                 \
   case NQ_: launch_post_nq<T, NQ_>(E, boxOut.get(), ghostOut.get(), smap.get(), wts.get(), Su, maskBits, s); break;
@@ -1486,7 +1525,7 @@ int Schwarz<T>::autotune(hipStream_t s)
   const int nv = tune_variants(TUNE_FDM, vals, 8);
   auto run = [&](int epw, float *o) {
     fdm_mfma_boxes(Nq, fdmPrecision, ras, E, u.get(), S16.get(), lam32.get(), helm32(), gmap.get(), o,
-                   ras ? nullptr : o + L, epw, s);
+                   ras ? nullptr : o + L, nullptr, nullptr, 1.f, epw, s);
   };
   run(4, ref.get());
   std::vector<float> hr(L + G), ho(L + G);

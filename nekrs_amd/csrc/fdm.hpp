@@ -71,10 +71,10 @@ struct Schwarz {
              bool poisson, double lambda0, double lambda1, hipStream_t s);
   // Su = smoothSchwarz(u): FDM solves on the extended boxes, overlap exchange,
   // gather-scatter, mask.  Su must not alias u (the RAS kernel reads the
-  // neighbours' u while writing its own Su).  Where takes_sub(): Su =
+  // neighbours' u while writing its own Su).  Where takes_sub() (FP32 vectors): Su =
   // scale * smoothSchwarz(u - sub), and diff = u - sub unless null (diff distinct
   // from u, sub and Su, for the same reason).
-  bool takes_sub() const { return std::is_same<T, float>::value && fdmPrecision == NRS_FDM_F32; }
+  bool takes_sub() const { return std::is_same<T, float>::value; }
   void apply(const T *u, T *Su, hipStream_t s, const T *sub = nullptr, T *diff = nullptr, T scale = T(1));
   void finish(T *Su, bool masked, hipStream_t s);
   // choose the matrix-core kernel's elements per wavefront for this level

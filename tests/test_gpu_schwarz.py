@@ -219,6 +219,30 @@ def test_mfma_smoother_vs_oracle(gpu, torch_mod, orc, fmt, S):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "fp16"])
+@pytest.mark.parametrize("S,N,degree", [("asm", 4, 1), ("ras", 4, 2), ("asm", 7, 4), ("ras", 7, 4)])
+def test_mfma_chebyshev_degrees_vs_oracle(gpu, torch_mod, orc, fmt, S, N, degree):
+    """One V-cycle with the residual formed inside the 16-bit boxes against the
+    oracle's emulation of the same roundings: a smoother application's bar for
+    each of the cycle's 2 degree of them."""
+    import oracle.mg as omg
+    torch = torch_mod
+    mg = gpu.BoxMesh(4, 3, 3, N, "kershaw", 0.3)
+    eg = gpu.Elliptic(mg, precon="multigrid", solver="fcg", levels=[N, 1], smoother=SM[("opt4", S)],
+                      cheby_degree=degree, fdmPrecision=FMTS[fmt])
+    mo = orc.BoxMesh(4, 3, 3, N, "kershaw", 0.3)
+    eo = orc.Elliptic(mo)
+    om = omg.MG(mo, [N, 1], T=np.float32, degree=degree, cheby="opt4", S=S, fmt=fmt)
+    r = np.random.default_rng(degree).uniform(-1, 1, eg.Nlocal)
+    r[eo.maskIds] = 0
+    r = eo.ogs.gs(r, "add")
+    z = torch.zeros(eg.Nlocal, dtype=torch.float64, device="cuda")
+    eg.preconditioner(dev(torch, r), z)
+    e = rel2(z.cpu().numpy(), om.apply(r))
+    print(fmt, S, N, degree, "rel", e)
+    assert e < 2 * degree * (2e-3 if fmt == "bf16" else 3e-4)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp16"])
 def test_mg_mfma_fcg_vs_oracle(gpu, torch_mod, orc, fmt):
     import oracle.mg as omg
     torch = torch_mod
