@@ -574,7 +574,8 @@ int nrs_batch_set_mode(nrs_batch *b, int mode);
  * the rows chunk c completes), keyed by dtype; NRS_TUNE_TOMBO = load schedule
  * {1: at use, 2: one plane ahead} of the pressure right-hand side's curl
  * kernels, type 0 = JW curl, 1 = the fused second curl + gradient (timed at
- * nrs_tombo_setup).
+ * nrs_tombo_setup; a tuned handle keeps its own choice, whatever a later setup
+ * of its key records, unless one is set by hand).
  * Keys are (kernel, N, type, floor(log2 Nelements)); a
  * setup with opts.autotune records the fastest variant whose result matches
  * the default's.  variant 0 = none recorded (the default is used). */

@@ -587,7 +587,7 @@ int nrs_set_variant(int kernel, int N, int type, int64_t Nelements, int variant)
   NRS_CHECK(kernel >= NRS_TUNE_AX && kernel <= NRS_TUNE_TOMBO, "set variant: unknown kernel");
   NRS_CHECK(N >= 1 && N <= 9 && type >= 0 && type < nrs::TUNE_TYPES && Nelements >= 1,
             "set variant: bad key");
-  nrs::set_tuned(kernel, N, type, Nelements, variant);
+  nrs::set_tuned(kernel, N, type, Nelements, variant, true);
   NRS_API_END
 }
 

@@ -17,6 +17,9 @@ struct nrs_tombo {
   nrs_ogs *ogsOp = nullptr;
   nrs::DevBuf<uint8_t> fx;
   int64_t fusedPairs = 0;
+  // load schedules of the JW curl and the right-hand-side kernel: the autotuner's
+  // for this handle's geometry and fusion (0: not tuned)
+  int sched[2] = {0, 0};
   int Nb = 0;                        // elements with at least one flux face
   nrs::DevBuf<int> bElem, bType;     // [Nb] element, [Nb][6] face boundary type
   nrs::DevBuf<double> bGeo;          // [Nb][6][Nq*Nq][4]: nx ny nz WSJ

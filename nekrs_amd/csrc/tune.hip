@@ -10,7 +10,8 @@ namespace nrs {
 
 namespace {
 
-// 0 = not tuned; N is 1..9
+// 0 = not tuned; N is 1..9; kByHand marks an entry the caller set
+constexpr int kByHand = 1 << 8;
 std::atomic<int> g_table[TUNE_KERNELS][10][TUNE_TYPES][TUNE_ECLASS];
 
 const int kAxVariants[] = {1, 2, 4};         // elements-per-block multipliers
@@ -46,11 +47,18 @@ int tune_eclass(int64_t E)
 int tuned(int kernel, int N, int type, int64_t E, int dflt)
 {
   if (!key_ok(kernel, N, type)) return dflt;
-  const int v = g_table[kernel][N][type][tune_eclass(E)].load(std::memory_order_relaxed);
+  const int v = g_table[kernel][N][type][tune_eclass(E)].load(std::memory_order_relaxed) & ~kByHand;
   return v ? v : dflt;
 }
 
-void set_tuned(int kernel, int N, int type, int64_t E, int variant)
+int tuned_by_hand(int kernel, int N, int type, int64_t E, int dflt)
+{
+  if (!key_ok(kernel, N, type)) return dflt;
+  const int v = g_table[kernel][N][type][tune_eclass(E)].load(std::memory_order_relaxed);
+  return (v & kByHand) ? v & ~kByHand : dflt;
+}
+
+void set_tuned(int kernel, int N, int type, int64_t E, int variant, bool byHand)
 {
   NRS_CHECK(key_ok(kernel, N, type), "tune: bad key");
   if (variant) {
@@ -60,7 +68,8 @@ void set_tuned(int kernel, int N, int type, int64_t E, int variant)
     for (int i = 0; i < nv; ++i) ok |= (vals[i] == variant);
     NRS_CHECK(ok, "tune: not a variant of this kernel");
   }
-  g_table[kernel][N][type][tune_eclass(E)].store(variant, std::memory_order_relaxed);
+  g_table[kernel][N][type][tune_eclass(E)].store(variant && byHand ? variant | kByHand : variant,
+                                                 std::memory_order_relaxed);
 }
 
 int tune_variants(int kernel, int *values, int max)

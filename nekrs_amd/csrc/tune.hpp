@@ -11,7 +11,10 @@
 //
 // Choices live in one process-wide table keyed by (kernel, order N, data
 // type, element-count class = floor(log2 E)); launches look their key up and
-// fall back to the default variant when nothing has been tuned.
+// fall back to the default variant when nothing has been tuned.  The load
+// schedules of the pressure right-hand side (TUNE_TOMBO) change the rounding and
+// depend on the handle's geometry and fusion: a tuned handle keeps its own and
+// reads from the table only what was set by hand.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,8 +29,10 @@ constexpr int TUNE_ECLASS = 32;    // floor(log2 E)
 int tune_eclass(int64_t E);
 // tuned variant of (kernel, N, type, E), or dflt when none is recorded
 int tuned(int kernel, int N, int type, int64_t E, int dflt);
+// the variant that the caller set for the key (nrs_set_variant), or dflt
+int tuned_by_hand(int kernel, int N, int type, int64_t E, int dflt);
 // record a variant (0 clears the entry)
-void set_tuned(int kernel, int N, int type, int64_t E, int variant);
+void set_tuned(int kernel, int N, int type, int64_t E, int variant, bool byHand = false);
 // number of variants of a kernel and their parameter values
 int tune_variants(int kernel, int *values, int max);
 

@@ -175,6 +175,36 @@ def test_load_schedules_agree(gpu, torch_mod, orc):
     assert rel(outs[1], outs[0]) <= 400 * np.finfo(np.float64).eps
 
 
+def test_tuned_handle_keeps_its_schedule(gpu, torch_mod, orc):
+    """A handle's load schedules, and so its bits, stay what they were when another of
+    the same order and size is tuned after it (stored factors: one plane ahead;
+    from the corners: at use); a second handle of the same form has the same
+    bits; a schedule set by hand is used by all until it is cleared."""
+    torch = torch_mod
+    N = 5
+    m, _ = meshes(gpu, orc, (8, 8, 8), N)
+    L = m.x.size
+    args = (*_rhs_inputs(torch, L, L, 4), 75.0, True)
+    a = gpu.PressureRhs(m)
+    first = a.compute(*args)
+    chosen = [gpu.tuned_variant("tombo", N, k, m.E) for k in ("curl", "rhs")]
+    b = gpu.PressureRhs(m, stored_geometry=True)
+    print("corners", chosen, "stored", [gpu.tuned_variant("tombo", N, k, m.E) for k in ("curl", "rhs")])
+    assert torch.equal(a.compute(*args), first)
+    assert torch.equal(gpu.PressureRhs(m).compute(*args), first)
+    try:
+        outs = []
+        for v in (1, 2):
+            gpu.set_variant("tombo", N, "curl", m.E, v)
+            gpu.set_variant("tombo", N, "rhs", m.E, v)
+            outs.append((a.compute(*args), b.compute(*args)))
+        assert not torch.equal(outs[0][0], outs[1][0]) and not torch.equal(outs[0][1], outs[1][1])
+    finally:
+        gpu.set_variant("tombo", N, "curl", m.E, 0)
+        gpu.set_variant("tombo", N, "rhs", m.E, 0)
+    assert torch.equal(a.compute(*args), first)
+
+
 @pytest.mark.parametrize("visc", [True, False])
 def test_face_fusion_bitwise(gpu, torch_mod, orc, visc):
     """The curl kernels' face fusion (N = 7, consecutive elements of a block of four)
