@@ -567,11 +567,13 @@ int nrs_batch_set_mode(nrs_batch *b, int mode);
 /* src/bench/fdm/benchmarkFDM.cpp:180-210)                                    */
 /* ------------------------------------------------------------------------- */
 /* Variants: NRS_TUNE_AX = elements-per-block multiplier {1, 2, 4} of the
- * operator kernel, keyed by dtype (nrs_dtype); NRS_TUNE_FDM = elements per
- * wavefront {1, 2, 4, 8} of the matrix-core Schwarz kernel, keyed by the
- * nrs_fdm_precision; NRS_TUNE_OPERATOR = element chunks {1, 2, 4, 8, 16} of
- * the solver operator (Ax of chunk c+1 overlapped with the gather-scatter of
- * the rows chunk c completes), keyed by dtype; NRS_TUNE_TOMBO = load schedule
+ * operator kernel, keyed by dtype (nrs_dtype; + 4 for the form that a multigrid
+ * level of a trilinear mesh uses, which takes the entry of dtype until it has
+ * its own); NRS_TUNE_FDM = elements per wavefront {1, 2, 4, 8} of the
+ * matrix-core Schwarz kernel, keyed by the nrs_fdm_precision;
+ * NRS_TUNE_OPERATOR = element chunks {1, 2, 4, 8, 16} of the solver operator
+ * (Ax of chunk c+1 overlapped with the gather-scatter of the rows chunk c
+ * completes), keyed by dtype; NRS_TUNE_TOMBO = load schedule
  * {1: at use, 2: one plane ahead} of the pressure right-hand side's curl
  * kernels, type 0 = JW curl, 1 = the fused second curl + gradient (timed at
  * nrs_tombo_setup; a tuned handle keeps its own choice, whatever a later setup

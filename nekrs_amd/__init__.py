@@ -562,12 +562,15 @@ def _tune_type(kernel, dtype):
         return FDM_PRECISIONS[dtype]
     if kernel == "tombo":
         return {"curl": 0, "rhs": 1}[dtype]
+    if kernel == "ax" and dtype.endswith("_corners"):
+        return 4 + DTYPES[dtype[:-len("_corners")]]
     return DTYPES[dtype]
 
 
 def tuned_variant(kernel, N, dtype, nelements):
     """Recorded launch variant for (kernel, N, type, E), 0 if none (nrs_tuned_variant).
-    type: a DTYPES name for "ax" and "op", an FDM_PRECISIONS name for "fdm", "curl" or
+    type: a DTYPES name for "ax" and "op" (with "_corners" for the "ax" of a multigrid
+    level that forms its geometry from the element corners), an FDM_PRECISIONS name for "fdm", "curl" or
     "rhs" for "tombo"."""
     t = _tune_type(kernel, dtype)
     v = C.c_int()

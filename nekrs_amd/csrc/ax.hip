@@ -375,9 +375,10 @@ static void launch_ax_trilin_nq(int mult, int E, const T *corners, const T *zw, 
 
 template <typename T>
 void launch_ax_trilin(int N, int E, const T *corners, const T *zw, const T *D, const T *l0, const T *l1,
-                      bool poisson, const T *q, T *Aq, const uint32_t *maskBits, hipStream_t s)
+                      bool poisson, const T *q, T *Aq, const uint32_t *maskBits, hipStream_t s, int mult)
 {
-  const int mult = tuned(TUNE_AX, N, dtype_of<T>::value, E, 1);
+  constexpr int type = dtype_of<T>::value;
+  if (!mult) mult = tuned(TUNE_AX, N, type + kTuneCorners, E, tuned(TUNE_AX, N, type, E, 1));
   switch (N + 1) {
 #define NRS_AXT_CASE(NQ_)                                                                          \
   case NQ_: launch_ax_trilin_nq<T, NQ_>(mult, E, corners, zw, D, l0, l1, poisson, q, Aq, maskBits, s); break;
@@ -389,10 +390,10 @@ void launch_ax_trilin(int N, int E, const T *corners, const T *zw, const T *D, c
 }
 template void launch_ax_trilin<double>(int, int, const double *, const double *, const double *,
                                        const double *, const double *, bool, const double *, double *,
-                                       const uint32_t *, hipStream_t);
+                                       const uint32_t *, hipStream_t, int);
 template void launch_ax_trilin<float>(int, int, const float *, const float *, const float *, const float *,
                                       const float *, bool, const float *, float *, const uint32_t *,
-                                      hipStream_t);
+                                      hipStream_t, int);
 
 // Ax with the face fusion (N = 7, M elements per block); fx [E] relative to q
 template <typename T, int M>

@@ -468,13 +468,14 @@ template void chunked_operator<float>(nrs_elliptic *, int, int, const float *, c
 template <typename T>
 int autotune_operator(nrs_elliptic *el, int N, int E, const T *ggeo, const T *D, const T *l0,
                       const T *l1, bool poisson, const uint32_t *maskBits, const nrs_ogs *ogs,
-                      hipStream_t s, const uint8_t *fx)
+                      hipStream_t s, const uint8_t *fx, const T *corners, const T *zw)
 {
   const int64_t L = (int64_t)E * (N + 1) * (N + 1) * (N + 1);
   DevBuf<T> q(L), ref(L), out(L);
   fill_pattern<T>(L, q.get(), s);
   auto run = [&](int k, T *o) {
-    chunked_operator<T>(el, N, E, ggeo, D, l0, l1, poisson, maskBits, ogs, q.get(), o, k, s, false, fx);
+    chunked_operator<T>(el, N, E, ggeo, D, l0, l1, poisson, maskBits, ogs, q.get(), o, k, s, false, fx,
+                        false, corners, zw);
   };
   run(1, ref.get());
   std::vector<T> hr(L), ho(L);
@@ -498,10 +499,12 @@ int autotune_operator(nrs_elliptic *el, int N, int E, const T *ggeo, const T *D,
 }
 template int autotune_operator<double>(nrs_elliptic *, int, int, const double *, const double *,
                                        const double *, const double *, bool, const uint32_t *,
-                                       const nrs_ogs *, hipStream_t, const uint8_t *);
+                                       const nrs_ogs *, hipStream_t, const uint8_t *, const double *,
+                                       const double *);
 template int autotune_operator<float>(nrs_elliptic *, int, int, const float *, const float *,
                                       const float *, const float *, bool, const uint32_t *,
-                                      const nrs_ogs *, hipStream_t, const uint8_t *);
+                                      const nrs_ogs *, hipStream_t, const uint8_t *, const float *,
+                                      const float *);
 
 // element part of the operator, all fields (no mask, no gather-scatter); three
 // fields go through the block kernel, which reads the geometric factors once

@@ -145,7 +145,8 @@ int operator_chunks(int N, int dtype, int64_t E);
 template <typename T>
 int autotune_operator(nrs_elliptic *el, int N, int E, const T *ggeo, const T *D, const T *l0,
                       const T *l1, bool poisson, const uint32_t *maskBits, const nrs_ogs *ogs,
-                      hipStream_t s, const uint8_t *fx = nullptr);
+                      hipStream_t s, const uint8_t *fx = nullptr, const T *corners = nullptr,
+                      const T *zw = nullptr);
 // Face fusion of an order-7 operator: from the masked ids [E*512] find the
 // pairs (e, e+1), e % nb != nb - 1, that share face i = N / i = 0 node for node
 // and hold the only two copies of each of those nodes (invDegree = 1/2, from

@@ -1210,9 +1210,12 @@ struct MGImpl final : MGSolver {
       // level operator launch variants (registerEllipticPreconditionerKernels.cpp:52-66)
       if (o.autotune) {
         autotune_ax<T>(l.N, l.E, l.ggeo, l.D, l.lam0.get(), l.lam1.get(), el->poisson, s);
+        const T *zw = l.corners ? l.zw.get() : nullptr;
+        if (l.corners)
+          autotune_ax<T>(l.N, l.E, l.ggeo, l.D, l.lam0.get(), l.lam1.get(), el->poisson, s, l.corners, zw);
         if (l.ogs->nChunks == nrs_elliptic::kOpChunks)
           autotune_operator<T>(el, l.N, l.E, l.ggeo, l.D, l.lam0.get(), l.lam1.get(), el->poisson,
-                               l.maskBits, l.ogs, s);
+                               l.maskBits, l.ogs, s, nullptr, l.corners, zw);
       }
       Nprev = l.N;
       levels.push_back(std::move(lp));

@@ -24,6 +24,10 @@ namespace nrs {
 
 enum TuneKernel { TUNE_AX = 0, TUNE_FDM = 1, TUNE_OP = 2, TUNE_TOMBO = 3, TUNE_KERNELS = 4 };
 constexpr int TUNE_TYPES = 8;      // data-type slots (nrs_dtype / nrs_fdm_precision codes)
+// TUNE_AX with the geometry formed from the element corners: dtype + this.  Bound by
+// vector instructions where the streaming form is bound by memory, so its variants
+// are timed by themselves; until they are, the streaming form's entry is used
+constexpr int kTuneCorners = 4;
 constexpr int TUNE_ECLASS = 32;    // floor(log2 E)
 
 int tune_eclass(int64_t E);
@@ -77,10 +81,11 @@ template <typename F> double time_launches(F &&f, hipStream_t s)
 }
 
 // Time every Ax variant on this operator's data (element count E, order N),
-// check that each gives the default variant's result bit for bit, record the
-// fastest.  Returns the chosen elements-per-block multiplier.
+// record the fastest whose result is within 400 eps of the default variant's.
+// With corners (and zw) the form that makes its geometry from them, under its own
+// key.  Returns the chosen variant.
 template <typename T>
 int autotune_ax(int N, int E, const T *ggeo, const T *D, const T *l0, const T *l1, bool poisson,
-                hipStream_t s);
+                hipStream_t s, const T *corners = nullptr, const T *zw = nullptr);
 
 }  // namespace nrs

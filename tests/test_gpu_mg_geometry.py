@@ -49,6 +49,54 @@ def test_corner_geometry_level_operators(gpu, torch_mod, N, prec):
         assert max(rel) < bar, rel
 
 
+@pytest.mark.parametrize("N", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_corner_variants(gpu, torch_mod, N, prec):
+    """Every elements-per-block variant of the corner form, set under its own key, on 63
+    elements, most often with a last block that is not full: the bars of the
+    level operators (the cofactors of much flatter elements than these cancel
+    more: 1.5e-13 in FP64 on a 7x7x1 box).  Order 1 is the coarse level."""
+    torch = torch_mod
+    mesh = gpu.BoxMesh(7, 3, 3, N, "kershaw", 0.3)
+    on, off = handles(gpu, mesh, [N, 1], prec, autotune=0)
+    t = "f64" if prec else "f32"
+    try:
+        for v in (1, 2, 4):
+            for n in (N, 1):
+                gpu.set_variant("ax", n, t + "_corners", mesh.E, v)
+            rel = level_ax_rel(torch, on, off, 2, torch.float64 if prec else torch.float32, N)
+            assert all(r < (1e-13 if prec else 1e-5) for r in rel), (v, rel)
+    finally:
+        for n in (N, 1):
+            gpu.set_variant("ax", n, t + "_corners", mesh.E, 0)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_setup_times_the_corner_form(gpu, torch_mod, prec):
+    """A tuned set-up records a variant for the form that each level runs: the corner
+    form under its own key where the mesh is trilinear (FP64 above order 7 streams),
+    none on a curved mesh, and the entry of the streaming form stays beside it."""
+    t = "f64" if prec else "f32"
+    orders, E = (9, 5, 1), 5 * 4 * 3
+    keys = [("ax", n, t + s, E) for n in orders for s in ("", "_corners")]
+
+    def recorded(mp):
+        for k in keys:
+            gpu.set_variant(*k, 0)
+        el = handles(gpu, gpu.BoxMesh(5, 4, 3, 9, mp, 0.3 if mp == "kershaw" else 0.0), list(orders), prec,
+                     autotune=1)[0]
+        del el
+        got = [gpu.tuned_variant(*k) for k in keys]
+        for k in keys:
+            gpu.set_variant(*k, 0)
+        return got
+
+    got = recorded("kershaw")
+    assert all(v in (1, 2, 4) for v in got[::2]), got
+    assert all((v == 0) if prec and n == 9 else v in (1, 2, 4) for n, v in zip(orders, got[1::2])), got
+    assert not any(recorded("sine")[1::2])
+
+
 def test_curved_mesh_unchanged(gpu, torch_mod):
     """Sine-mapped nodes are not trilinear: the option has no effect."""
     torch = torch_mod
