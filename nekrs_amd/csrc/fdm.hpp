@@ -78,8 +78,9 @@ struct Schwarz {
   void apply(const T *u, T *Su, hipStream_t s, const T *sub = nullptr, T *diff = nullptr, T scale = T(1));
   void finish(T *Su, bool masked, hipStream_t s);
   // choose the matrix-core kernel's elements per wavefront for this level
-  // (FP32 vectors with BF16/FP16 operators; otherwise nothing to tune); returns it
-  int autotune(hipStream_t s);
+  // (FP32 vectors with BF16/FP16 operators; otherwise nothing to tune), timed with
+  // the difference u - sub formed in the boxes or without; returns it
+  int autotune(bool difference, hipStream_t s);
 };
 
 }  // namespace nrs

@@ -1205,7 +1205,9 @@ struct MGImpl final : MGSolver {
           l.betasDown = opt4_betas<T>(l.degDown);
           l.betasUp = opt4_betas<T>(l.degUp);
         }
-        if (o.autotune && l.schwarz) l.schwarz->autotune(s);
+        // the 4th-kind recurrence forms all residuals but the first in the boxes, the
+        // first-kind only the one of a non-zero start
+        if (o.autotune && l.schwarz) l.schwarz->autotune(cheby == CHEBY_OPT4, s);
       }
       // level operator launch variants (registerEllipticPreconditionerKernels.cpp:52-66)
       if (o.autotune) {

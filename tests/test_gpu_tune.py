@@ -105,6 +105,43 @@ def test_fdm_variants_bitwise(gpu, torch_mod, smoother, fmt):
             gpu.set_variant("fdm", N, fmt, E, 0)
 
 
+@pytest.mark.parametrize("smoother,fmt,N", [("opt4chebyshev+ras", "bf16", 7), ("opt4chebyshev+asm", "fp16", 7),
+                                            ("opt4chebyshev+asm", "bf16", 4), ("opt4chebyshev+ras", "fp16", 9)])
+def test_fdm_variants_bitwise_in_the_cycle(gpu, torch_mod, smoother, fmt, N):
+    """The box solves that form the residual as they load, and keep it, give the same
+    V-cycle bit for bit with every variant, and with the one that the set-up
+    times and records."""
+    torch = torch_mod
+    m = gpu.BoxMesh(5, 4, 3, N, "kershaw", 0.2)
+    kw = dict(solver="fcg", precon="multigrid", smoother=smoother, cheby_degree=3, levels=[N, 3, 1],
+              fdmPrecision=gpu.FDM_PRECISIONS[fmt], useGraphs=0)
+    el = gpu.Elliptic(m, autotune=0, **kw)
+    r = torch.from_numpy(np.random.default_rng(3).uniform(-1, 1, m.Nlocal)).cuda()
+    keys = [("fdm", n, fmt, m.E) for n in (N, 3)]
+    outs = []
+    try:
+        for epw in (0, 1, 2, 4, 8):
+            for k in keys:
+                gpu.set_variant(*k, epw)
+            z = torch.full_like(r, float("nan"))
+            el.preconditioner(r, z)
+            torch.cuda.synchronize()
+            outs.append(z)
+        assert torch.isfinite(outs[0]).all()
+        for z in outs[1:]:
+            assert torch.equal(z, outs[0])
+        gpu.Elliptic(m, autotune=1, **kw)
+        assert all(gpu.tuned_variant(*k) in (1, 2, 4, 8) for k in keys)
+    finally:
+        for k in keys:
+            gpu.set_variant(*k, 0)
+        for n in (N, 3, 1):
+            for t in ("f64", "f32", "f32_corners"):
+                gpu.set_variant("ax", n, t, m.E, 0)
+        for t in ("f64", "f32"):
+            gpu.set_variant("op", N, t, m.E, 0)
+
+
 def test_autotune_setup_records_and_solves(gpu, torch_mod, orc):
     import oracle.mg as omg
     torch = torch_mod
