@@ -239,12 +239,19 @@ __global__ void cheby4_dir_kernel(int64_t n, T beta, T rC, T dC, T betaLast, con
   }
 }
 
-// y = a x (+ b y when b != 0)
+// y = a x (+ b y when b != 0), x not y
 template <typename T>
 __global__ void axpby_kernel(int64_t n, T a, const T *__restrict__ x, T b, T *__restrict__ y)
 {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     y[i] = (b == T(0)) ? a * x[i] : a * x[i] + b * y[i];
+}
+
+// y = a y
+template <typename T> __global__ void scale_kernel(int64_t n, T a, T *__restrict__ y)
+{
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    y[i] = a * y[i];
 }
 
 // y = w .* x (in place when y == x)
@@ -660,7 +667,10 @@ struct MGImpl final : MGSolver {
       NRS_LAUNCH_CHECK();
     }
     smootherS(l, b ? tmp : a, Su, s);
-    if (scale != T(1)) k_axpby<T>(l.L, scale, Su, T(0), Su, s);
+    if (scale != T(1)) {
+      scale_kernel<T><<<kgrid(l.L), KB, 0, s>>>(l.L, scale, Su);
+      NRS_LAUNCH_CHECK();
+    }
     return tmp;
   }
 
