@@ -51,14 +51,14 @@ def test_ax_vs_oracle(gpu, torch_mod, orc, N, T, kind):
     assert rel(host(Aq), ref) < tol
 
 
-@pytest.mark.parametrize("N", [1, 2, 4, 5, 6, 7])
+@pytest.mark.parametrize("N", NS)
 @pytest.mark.parametrize("T", [np.float64, np.float32])
 @pytest.mark.parametrize("extra", [0, 1])
 def test_ax_at_the_load_ahead_line(gpu, torch_mod, orc, N, T, extra):
     """The launch loads every plane's factors ahead up to E (N+1)^2 = 65536 threads
     and one plane ahead beyond: the last mesh of one form and the first of the
-    other (a last block of fewer elements in both), against the oracle with the
-    bars of test_ax_vs_oracle."""
+    other (a last block of fewer elements in most; FP64 above order 7 has one form),
+    against the oracle with the bars of test_ax_vs_oracle."""
     torch = torch_mod
     E = 65536 // (N + 1) ** 2 + extra
     m = orc.BoxMesh(E, 1, 1, N, "kershaw", 0.3)
@@ -125,6 +125,29 @@ def test_block_ax_golden(gpu, torch_mod, golden, N):
                  Aq, L, L, E)
     torch.cuda.synchronize()
     assert rel(host(Aq), g[k + "_Aq"]) < 1e-12
+
+
+@pytest.mark.parametrize("N", NS)
+def test_block_ax_every_order(gpu, torch_mod, orc, N):
+    """Three fields with coefficient fields of their own against the single-field oracle,
+    FP64 1e-12: orders 8 and 9 read D from LDS every plane, order 9 has a smaller
+    block, and 37 elements leave the last block of every order unfilled."""
+    torch = torch_mod
+    rng = np.random.default_rng(200 + N)
+    m = orc.BoxMesh(37, 1, 1, N, "kershaw", 0.3)
+    L = m.E * m.Np
+    off, loff = L + 24, L + 8
+    q, l0, l1 = rng.uniform(-1, 1, 3 * off), rng.uniform(0.5, 2, 3 * loff), rng.uniform(0, 10, 3 * loff)
+    Aq = torch.full((3 * off,), 7.0, dtype=torch.float64, device="cuda")
+    gpu.block_ax(N, dev(torch, m.ggeo), dev(torch, m.D.ravel()), dev(torch, l0), dev(torch, l1), dev(torch, q), Aq,
+                 off, loff, m.E)
+    torch.cuda.synchronize()
+    got = host(Aq).reshape(3, off)
+    for f in range(3):
+        ref = orc.ax(N, m.ggeo, m.D, q[f * off:f * off + L].copy(), lambda0=l0[f * loff:f * loff + L].copy(),
+                     lambda1=l1[f * loff:f * loff + L].copy(), poisson=False)
+        assert rel(got[f, :L], ref) < 1e-12, f
+    assert np.all(got[:, L:] == 7.0)
 
 
 @pytest.mark.parametrize("N", [1, 3, 7, 9])

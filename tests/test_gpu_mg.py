@@ -270,20 +270,24 @@ def test_mg_schedule_degrees_vs_oracle(gpu, torch_mod, orc):
 
 
 @pytest.mark.parametrize("mgp,smoother", [(0, "opt4chebyshev+ras"), (1, "chebyshev+jacobi")])
-def test_vcycle_from_level_operations(gpu, torch_mod, orc, mgp, smoother):
+@pytest.mark.parametrize("levels", [(5, 3, 1), (4, 2, 1), (5, 4, 1), (4, 3, 1), (5, 2, 1), (3, 2, 1), (7, 6, 5)])
+def test_vcycle_from_level_operations(gpu, torch_mod, orc, mgp, smoother, levels):
     """A V-cycle composed by hand from the per-level operations
     (nrs_elliptic_mg_level: smooth, residual, coarsen, prolongate, as
     MGSolver_t::runVcycle, MGSolver.cpp:167-193, calls them) gives the library's
-    preconditioner bit for bit; the level Ax and residual agree with each other."""
+    preconditioner bit for bit; the level Ax and residual agree with each other.
+    The cycle's coarsening takes the residual, the weights and the mask as it loads
+    and stores: all pairs of orders up to 5 but (5, 1), and two above."""
     torch = torch_mod
-    mesh = gpu.BoxMesh(3, 3, 2, 5, "kershaw", 0.3)
-    el = gpu.Elliptic(mesh, precon="multigrid", solver="fcg", levels=[5, 3, 1], smoother=smoother,
+    N = levels[0]
+    mesh = gpu.BoxMesh(3, 3, 2, N, "kershaw", 0.3)
+    el = gpu.Elliptic(mesh, precon="multigrid", solver="fcg", levels=list(levels), smoother=smoother,
                       cheby_degree=2, coarse="smooth_jacobi", mgPrecision=mgp, fdmPrecision=0,
                       autotune=0)
     T = torch.float32 if mgp == 0 else torch.float64
     lv, _ = el.mg_info()
     n = [l["Nlocal"] for l in lv]
-    eo = orc.Elliptic(orc.BoxMesh(3, 3, 2, 5, "kershaw", 0.3))
+    eo = orc.Elliptic(orc.BoxMesh(3, 3, 2, N, "kershaw", 0.3))
     r = dev(torch, assembled_random(eo, 9))
     z = torch.zeros_like(r)
     el.preconditioner(r, z)

@@ -286,3 +286,26 @@ def test_fp32_boxes_every_order(gpu, torch_mod, orc, N, S):
     got = out.cpu().numpy()
     assert rel(got, ref) < 2e-5, rel(got, ref)
     assert np.all(got[L.el.maskIds] == 0)
+
+
+@pytest.mark.parametrize("S", ["asm", "ras"])
+def test_fp32_boxes_order_1(gpu, torch_mod, orc, S):
+    """The box edge of 4 (one tile of 16 rows, one contraction step): a smoothed
+    coarse level of order 1, with the bar of the other orders."""
+    import oracle.mg as omg
+    torch = torch_mod
+    shape = (5, 4, 3)
+    eg = gpu.Elliptic(gpu.BoxMesh(*shape, 2, "kershaw", 0.3), precon="multigrid", solver="fcg", levels=[2, 1],
+                      smoother=SM[("opt4", S)], cheby_degree=3, coarse="smooth", mgPrecision=0)
+    L = omg.MG(orc.BoxMesh(*shape, 2, "kershaw", 0.3), [2, 1], T=np.float64, degree=3, cheby="opt4", S=S,
+               coarse="smooth").levels[1]
+    x = np.random.default_rng(1).uniform(-1, 1, L.E * L.Np)
+    x[L.el.maskIds] = 0
+    x = L.el.ogs.gs(x, "add").astype(np.float32)
+    ref = L.schwarz.apply(x.astype(np.float64))
+    assert np.max(np.abs(ref)) > 0
+    out = torch.zeros(L.E * L.Np, dtype=torch.float32, device="cuda")
+    eg.mg_smoother(1, dev(torch, x), out)
+    got = out.cpu().numpy()
+    assert rel(got, ref) < 2e-5, rel(got, ref)
+    assert np.all(got[L.el.maskIds] == 0)

@@ -268,6 +268,27 @@ def test_block_three_fields_vs_oracle(gpu, torch_mod, orc, N, lam1):
     assert rel(host(x), xo) <= 1e-8
 
 
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+def test_block_operator_every_order(gpu, torch_mod, orc, N):
+    """The three-field operator with constant coefficients, its Dirichlet mask stored by the
+    element kernel, at every order and on 44 elements (a last block that is not
+    full at most orders): 1e-12 of the oracle's on each field, zero at masked nodes."""
+    torch = torch_mod
+    shape = (11, 2, 2)
+    eg = gpu.Elliptic(gpu.BoxMesh(*shape, N, "kershaw", 0.3), lambda0=1.3, lambda1=2.5, poisson=False, nfields=3,
+                      precon="jacobi", autotune=0)
+    mo = orc.BoxMesh(*shape, N, "kershaw", 0.3)
+    eo = orc.Elliptic(mo, 1.3, 2.5, False)
+    L = mo.Nlocal
+    q = np.random.default_rng(N).uniform(-1, 1, 3 * L)
+    Aq = torch.zeros(3 * L, dtype=torch.float64, device="cuda")
+    eg.operator(dev(torch, q), Aq)
+    got = host(Aq).reshape(3, L)
+    for f in range(3):
+        assert rel(got[f], eo.operator(q[f * L:(f + 1) * L])) < 1e-12
+    assert np.all(got[:, eo.maskIds] == 0)
+
+
 def test_block_rejects_two_fields(gpu):
     m = gpu.BoxMesh(2, 2, 2, 3)
     with pytest.raises(gpu.NrsError):

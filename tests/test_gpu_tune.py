@@ -69,6 +69,31 @@ def test_ax_variants_vs_oracle(gpu, torch_mod, orc, N, T, mult):
         gpu.set_variant("ax", N, tname, len(elist), 0)
 
 
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("T", [np.float64, np.float32])
+@pytest.mark.parametrize("many", [False, True])
+def test_ax_variants_constant_coefficients(gpu, torch_mod, orc, N, T, many):
+    """Every variant at every order with constant coefficients, which on few elements
+    loads all planes' factors ahead and beyond 65536 threads one plane ahead
+    (FP64 above order 7 always), against the oracle with the bars above."""
+    torch = torch_mod
+    E = 65536 // (N + 1) ** 2 + 1 if many else 53
+    m = orc.BoxMesh(E, 1, 1, N, "kershaw", 0.3)
+    q = np.random.default_rng(N).uniform(-1, 1, E * m.Np)
+    ref = orc.ax(N, m.ggeo.astype(T), m.D.astype(T), q.astype(T), lambda0=1.3, lambda1=2.0, poisson=False, dtype=T)
+    tname = "f64" if T == np.float64 else "f32"
+    args = [dev(torch, a.astype(T)) for a in (m.ggeo, m.D.ravel(), q)]
+    l0, l1 = (dev(torch, np.array([c], dtype=T)) for c in (1.3, 2.0))
+    try:
+        for mult in (1, 2, 4):
+            gpu.set_variant("ax", N, tname, E, mult)
+            Aq = torch.full_like(args[2], float("nan"))
+            gpu.ax(N, *args, Aq, lambda0=l0, lambda1=l1, poisson=False)
+            assert rel(Aq.cpu().numpy(), ref) < (1e-12 if T == np.float64 else 2e-5), mult
+    finally:
+        gpu.set_variant("ax", N, tname, E, 0)
+
+
 def test_set_variant_rejects_unknown(gpu):
     with pytest.raises(gpu.NrsError):
         gpu.set_variant("ax", 3, "f64", 100, 3)
