@@ -566,8 +566,8 @@ int nrs_batch_set_mode(nrs_batch *b, int mode);
 /* variants at setup: src/bench/axHelm/benchmarkAx.cpp:268-383,               */
 /* src/bench/fdm/benchmarkFDM.cpp:180-210)                                    */
 /* ------------------------------------------------------------------------- */
-/* Variants: NRS_TUNE_AX = elements-per-block multiplier {1, 2, 4} of the
- * operator kernel, keyed by dtype (nrs_dtype; + 4 for the form that a multigrid
+/* Variants: NRS_TUNE_AX = block shape {1, 2, 4} of the operator kernel (whole
+ * elements that fill its waves, at orders 1..4 and 7 in that proportion), keyed by dtype (nrs_dtype; + 4 for the form that a multigrid
  * level of a trilinear mesh uses, which takes the entry of dtype until it has
  * its own); NRS_TUNE_FDM = elements per wavefront {1, 2, 4, 8} of the
  * matrix-core Schwarz kernel, keyed by the nrs_fdm_precision;

@@ -599,7 +599,8 @@ void Amg::apply(const double *b, double *z, double *tmp, hipStream_t s)
 // ------------------------------------------------------------------ fixed-iteration PCG
 //
 // `maxit` AMG-preconditioned CG iterations from x = 0 on device scalars, the
-// scalar steps of pcg_* (linalg.hip) with its sums in its order.  Each sum's
+// scalar steps of pcg_* (linalg.hip); the sums are grouped over fewer blocks (8
+// entries a thread, for every block adds their partials again).  Each sum's
 // block partials are added by every block of the kernel that needs the value
 // (a few kilobytes from L2) instead of by a one-block launch of its own, the
 // first iteration takes p = z and x = alpha z as they are, and the last one

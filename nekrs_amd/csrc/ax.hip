@@ -49,8 +49,8 @@ template <int NQ> __device__ __forceinline__ void plane_sync()
   }
 }
 
-// Elements per block of a launch variant (1, 2, 4): whole elements that fill the
-// lanes of the block's waves.  An element of NQ^2 threads leaves lanes idle at
+// Elements per block of a launch variant (1, 2, 4; elements in proportion at orders 1
+// to 4 and 7 only): whole elements that fill the lanes of the block's waves.  An element of NQ^2 threads leaves lanes idle at
 // most orders: order 5 ran 72 threads in two waves (56 %), order 9 100 in two
 // (78 %); the first entry of every order fills at least 94 %.  Larger blocks than
 // these would cap the registers of the high orders.  Order 7 is one element per
@@ -443,7 +443,7 @@ template void launch_ax_fused<float>(int, int, const float *, const float *, con
                                      const float *, bool, const float *, float *, const uint32_t *,
                                      const uint8_t *, hipStream_t, int);
 
-// elements-per-block multiplier: the autotuner's choice for (N, type), else 1
+// block shape: the autotuner's choice for (N, type), else variant 1
 template <typename T>
 void launch_ax(int N, int E, const int *elist, const T *ggeo, const T *D, const T *l0, const T *l1,
                bool poisson, bool lfield, const T *q, T *Aq, const uint32_t *maskBits,
@@ -472,12 +472,14 @@ template void launch_ax<float>(int, int, const int *, const float *, const float
 // the geometric factors are read once for the three fields.
 // -------------------------------------------------------------------------------------
 // Same scheme as ax_kernel: one (i,j) column per lane, the k-pencils of q and
-// of the result in registers over unrolled planes, r/s contractions through LDS slabs, geometric factors prefetched one
-// plane ahead and shared by the three fields, blocks of whole elements that fill
-// their waves (AxShape), the Dirichlet mask in the store (maskBits, optional).
-// HBM-bound in the count of bytes, held back by two waves per SIMD (registers):
-// order 5, 5814 curved elements 57.8 -> 33 us (131 MB, 3.9 TB/s), and no mask pass.
-// coefficient fields at order 9: smaller blocks, for the registers
+// of the result in registers over unrolled planes, r/s contractions through LDS
+// slabs, geometric factors prefetched one plane ahead and shared by the three
+// fields, blocks of whole elements that fill their waves, the Dirichlet mask in
+// the store (maskBits, optional).  HBM-bound in the count of bytes, held back by two
+// waves per SIMD (registers): order 5, 5814 curved elements 57.8 -> 33 us (131 MB,
+// 3.9 TB/s), and no mask pass.
+
+// AxShape's blocks, smaller ones with coefficient fields at order 9 for their registers
 template <int NQ, bool LFIELD> using BlockAxShape = AxShape<NQ, (NQ == 10 && LFIELD) ? 2 : 1>;
 template <int NQ, bool LFIELD>
 __global__ void __launch_bounds__((BlockAxShape<NQ, LFIELD>::THREADS), LFIELD ? 1 : 2)

@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(256, FdmF32Cfg<NQ>::WAVES_PER_EU) void fdm_f32_kern
   auto as_is = [](float (&)[NT][KS]) {};
   // T3[p][n][m] *= invL as the next contraction reads it (KS values a row and
   // lane against four where the sums come out).  1 / d in FP64: the hardware's
-  // estimate and one Newton step (error below 1e-13), rounded once to FP32.
+  // estimate and one Newton step (relative error 2^-48, measured), rounded once to FP32.
   auto by_invL = [&](float (&a)[NT][KS]) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {

@@ -11,7 +11,7 @@ template <typename T>
 void launch_ax(int N, int E, const int *elist, const T *ggeo, const T *D, const T *l0, const T *l1,
                bool poisson, bool lfield, const T *q, T *Aq, const uint32_t *maskBits,
                hipStream_t s);
-// the same with an explicit elements-per-block multiplier (1, 2 or 4)
+// the same with an explicit block shape (variant 1, 2 or 4)
 template <typename T>
 void launch_ax_variant(int N, int mult, int E, const int *elist, const T *ggeo, const T *D,
                        const T *l0, const T *l1, bool poisson, bool lfield, const T *q, T *Aq,

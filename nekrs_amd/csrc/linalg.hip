@@ -193,13 +193,14 @@ update_rx_kernel(int64_t n, const double *__restrict__ w, const double *__restri
   write_partials<1>(v, partials);
 }
 
-// ---- PCG without a preconditioner or with Jacobi in five launches an iteration
-// beside the operator's: where the vectors are short an iteration is as long as
+// ---- PCG without a preconditioner or with Jacobi in four launches an iteration
+// beside the operator's two: where the vectors are short an iteration is as long as
 // its launches (8^3 elements, order 7: 9 launches, 40 us; now 6, 32 us).  The preconditioned
 // residual z = invDiag .* r is formed where it is read (rounded on its own, as
 // a stored z is), <r,z>_w is summed by the kernel that updates r, and alpha's
 // partials are added by every block of that kernel instead of by a launch of
-// their own.  The same sums in the same order: the same iterates bit for bit.
+// their own.  The sums and their order are those of the kernels replaced: the same
+// iterates bit for bit over the same grid.
 template <int MODE>
 __global__ void update_p_direct_kernel(int64_t n, const double *__restrict__ invDiag, const double *__restrict__ r,
                                        double *__restrict__ p, const double *__restrict__ scal)

@@ -14,7 +14,7 @@ namespace {
 constexpr int kByHand = 1 << 8;
 std::atomic<int> g_table[TUNE_KERNELS][10][TUNE_TYPES][TUNE_ECLASS];
 
-const int kAxVariants[] = {1, 2, 4};         // elements-per-block multipliers
+const int kAxVariants[] = {1, 2, 4};         // block shapes (AxShape)
 const int kFdmVariants[] = {1, 2, 4, 8};     // elements per wavefront
 const int kOpVariants[] = {1, 2, 4, 8, 16};  // operator chunks (Ax overlapped with gs)
 const int kTomboVariants[] = {1, 2};        // pressure-rhs volume kernels: inputs loaded at use / one plane ahead
