@@ -1037,8 +1037,8 @@ __global__ __launch_bounds__(256) void fdm_mfma_kernel(
 // invL) -> T4[i][p][n] -> T5[j][i][p] -> out[k][j][i].  FP32 operands and sums, as in the
 // one-thread-per-pencil form this replaced, which spent its time waiting for
 // scalar loads of the operators (100 each in six phases).  Order 7, 8000
-// elements: 47.3 -> 33 us a launch (counters: matrix cores busy 45 % of it, VALU
-// 25 %, the rest the loads at the start of each wave; a persistent wave that
+// elements: 47.3 -> 33 us a launch (counters: matrix cores busy 38 % of it, VALU
+// 23 %, the rest the loads at the start of each wave; a persistent wave that
 // loads the next element ahead, 1 to 5 blocks per CU, was 5-60 % slower).
 // SUB: the boxes of u - sub, the difference kept in diff where that is not null;
 // results times scale.  A Chebyshev step's residual update and first scaling then
